@@ -1,5 +1,6 @@
 // Smoothed-aggregation AMG V-cycle on the device, with the hierarchy's matrix values
-// in FP64 or FP32.
+// in FP64 or FP32 (most solves with an operator in stencil form take mg.hpp's levels
+// instead: AmgPrecond's second constructor).
 //
 // One application is one V-cycle from a zero initial guess: on every level but the
 // coarsest, npre weighted-Jacobi sweeps (omega = 0.8; the first is x = omega D^-1 b),
@@ -20,6 +21,7 @@
 
 #include "batch.hpp"
 #include "krylov.hpp"
+#include "mg.hpp"
 #include "stencil.hpp"
 
 namespace cuibm {
@@ -290,11 +292,6 @@ template <class V, class X>
 struct AmgDev {
     std::vector<AmgLevelDev<V, X>> lv;
     DArray<V> coarse_inv;
-    DArray<float> fine_dinv32;  // FP32 D^-1 of the stencil finest level (FP32 V-cycle)
-    // FP64 deflation of the pinned constant mode (FP32 V-cycle on a stencil finest level):
-    // partial sums, c, and 1 / sum over the pins of area * (A 1)
-    DArray<double> defl_part, defl_c;
-    double inv_wa = 0;
     int nc = 0, ld = 0;
     AmgParams prm;
     bool use_fine = false;  // finest level in stencil form (fused kernels)
@@ -340,15 +337,9 @@ struct AmgDev {
             L.xt.alloc(L.n);
             L.r.alloc(L.n);
         }
-        if (use_fine && !kVec64) {
-            fine_dinv32.alloc(lv[0].n);
-            launch_to_float(fine_dinv32.p(), fine.dinv, lv[0].n, s);
-            fine.dinv32 = fine_dinv32.p();
-        }
         nc = h.back().A.n;
         if (nc > 6144) throw Error("AMG coarsening stalled at " + std::to_string(nc) + " unknowns", ERR_GENERIC);
-        std::vector<double> inv = dense_inverse(h.back().A);
-        if (fine.defl) deflate_coarse(inv, nc);
+        const std::vector<double> inv = dense_inverse(h.back().A);
         ld = (nc + 3) & ~3;  // row stride, zero-padded to a multiple of 4 values
         std::vector<V> invt((size_t)nc * ld, V(0));
         for (int i = 0; i < nc; i++)
@@ -357,69 +348,21 @@ struct AmgDev {
         CUIBM_HIP(hipStreamSynchronize(s));
     }
 
-    // With the finest level deflated (the FP32 V-cycle), the coarsest operator is still
-    // weakly pinned: its inverse has one eigenvalue 1/mu far above the others, whose
-    // eigenvector is close to the constant, and an FP32 copy of it (and FP32 level vectors
-    // holding its huge component) would drown everything else in rounding. The constant
-    // mode is already carried in FP64 by the finest-level deflation, so that component is
-    // removed here (Wielandt deflation, in FP64, before the FP32 copy):
-    //   inv <- inv - sigma v u^T / (u^T v),
-    // with sigma, v, u the dominant eigenvalue and right / left eigenvectors of inv by
-    // power iteration (the gap to the next eigenvalue makes a few iterations exact).
-    static void deflate_coarse(std::vector<double> &inv, int n) {
-        auto power = [&](bool left) {
-            std::vector<double> x(n, 1.0), y(n);
-            for (int it = 0; it < 60; it++) {
-                for (int i = 0; i < n; i++) {
-                    double a = 0;
-                    for (int j = 0; j < n; j++) a += (left ? inv[(size_t)j * n + i] : inv[(size_t)i * n + j]) * x[j];
-                    y[i] = a;
-                }
-                double nrm = 0;
-                for (double v : y) nrm += v * v;
-                nrm = std::sqrt(nrm);
-                if (!(nrm > 0)) break;
-                double diff = 0;
-                for (int i = 0; i < n; i++) {
-                    const double v = y[i] / nrm;
-                    diff = std::max(diff, std::fabs(v - x[i]));
-                    x[i] = v;
-                }
-                if (diff < 1e-15) break;
-            }
-            return x;
-        };
-        const std::vector<double> v = power(false), u = power(true);
-        double uv = 0, uiv = 0;
-        for (int i = 0; i < n; i++) {
-            uv += u[i] * v[i];
-            double a = 0;
-            for (int j = 0; j < n; j++) a += inv[(size_t)i * n + j] * v[j];
-            uiv += u[i] * a;
-        }
-        if (!(std::fabs(uv) > 1e-12)) return;  // no separated mode to remove
-        const double sigma = uiv / uv;
-        for (int i = 0; i < n; i++)
-            for (int j = 0; j < n; j++) inv[(size_t)i * n + j] -= sigma * v[i] * u[j] / uv;
-    }
-
-    // the preconditioner: one V-cycle from x = 0 on the FP64 Krylov vectors b and x;
-    // weighted: the deflation's partial sums of b are already in defl_part
-    void apply(const double *b, double *x, hipStream_t s, bool weighted = false) {
-        const X w = (X)prm.omega;
-        if (use_fine && prm.npre == 2 && prm.npost == 2 && lv.size() > 1) {
-            // stencil finest level: x2 -> xt and r -> r, restriction, coarse cycle,
-            // prolongation into xt, both post-sweeps straight into x
-            AmgLevelDev<V, X> &L = lv[0], &C = lv[1];
-            if (fine.defl && !weighted) launch_p5_wdot(fine, b, defl_part.p(), s);
-            launch_p5_pre(fine, w, b, L.xt.p(), L.r.p(), s, probe);
-            launch_csr_op<V, X, OP_SPMV>(L.lanesR, L.R, L.r.p(), nullptr, nullptr, C.b.p(), X(0), s, stop);
-            vcycle(1, C.b.p(), C.x.p(), s);
-            launch_csr_op<V, X, OP_PROLONG>(L.lanesP, L.P, C.x.p(), nullptr, nullptr, L.xt.p(), X(0), s, stop);
-            launch_p5_sweep2(fine, w, L.xt.p(), b, x, s);
-            return;
-        }
+    // the preconditioner: one V-cycle from x = 0 on the FP64 Krylov vectors b and x
+    void apply(const double *b, double *x, hipStream_t s) {
         if constexpr (kVec64) {
+            const X w = (X)prm.omega;
+            if (use_fine && prm.npre == 2 && prm.npost == 2 && lv.size() > 1) {
+                // stencil finest level: x2 -> xt and r -> r, restriction, coarse cycle,
+                // prolongation into xt, both post-sweeps straight into x
+                AmgLevelDev<V, X> &L = lv[0], &C = lv[1];
+                launch_p5_pre(fine, w, b, L.xt.p(), L.r.p(), s, probe);
+                launch_csr_op<V, X, OP_SPMV>(L.lanesR, L.R, L.r.p(), nullptr, nullptr, C.b.p(), X(0), s, stop);
+                vcycle(1, C.b.p(), C.x.p(), s);
+                launch_csr_op<V, X, OP_PROLONG>(L.lanesP, L.P, C.x.p(), nullptr, nullptr, L.xt.p(), X(0), s, stop);
+                launch_p5_sweep2(fine, w, L.xt.p(), b, x, s);
+                return;
+            }
             vcycle(0, b, x, s);
         } else {
             AmgLevelDev<V, X> &L = lv[0];
@@ -509,6 +452,7 @@ struct AmgPrecond::Impl {
     std::vector<HostAmgLevel> host;
     KernelProbe probe;
     RefreshData rf;
+    std::unique_ptr<TensorMg> mg;  // in place of the others
     template <class F>
     void each(F f) {
         f(d64);
@@ -517,14 +461,18 @@ struct AmgPrecond::Impl {
     }
 };
 
-KernelProbe &AmgPrecond::pre_probe() { return im_->probe; }
+KernelProbe &AmgPrecond::pre_probe() { return im_->mg ? im_->mg->probe() : im_->probe; }
+TensorMg *AmgPrecond::tensor() const { return im_->mg.get(); }
 
 static void refresh_setup(RefreshData &rf, const std::vector<HostAmgLevel> &host, hipStream_t s);
 
+static void check_precision(int p) {
+    if (p != 64 && p != 32 && p != 3264) throw Error("AMG precision must be 64, 32 or 3264", ERR_ARGUMENT);
+}
+
 AmgPrecond::AmgPrecond(const HCsr &A, const AmgParams &p, hipStream_t s, const P5Dev *fine)
     : im_(new Impl), prm_(p) {
-    if (p.precision != 64 && p.precision != 32 && p.precision != 3264)
-        throw Error("AMG precision must be 64, 32 or 3264", ERR_ARGUMENT);
+    check_precision(p.precision);
     // a hierarchy set up again on the device for moving bodies is built on a padded
     // pattern that the moved body's rows keep to (the padding entries are zeros, so the
     // values, aggregates and levels are those of A's own hierarchy)
@@ -532,7 +480,7 @@ AmgPrecond::AmgPrecond(const HCsr &A, const AmgParams &p, hipStream_t s, const P
     HCsr padded;
     if (pad) padded = pad_pattern(A, p.pad_nx, p.pad_margin);
     im_->host = amg_build(pad ? padded : A, p.coarse_max, p.max_levels, p.scale0, p.fused_restriction);
-    fine_ = fine != nullptr && im_->host.size() > 1 && p.npre == 2 && p.npost == 2;
+    fine_ = fine != nullptr && p.precision != 32 && im_->host.size() > 1 && p.npre == 2 && p.npost == 2;
     if (fine_) {
         if (fine->nx * fine->ny != A.n) throw Error("stencil and matrix sizes differ", ERR_ARGUMENT);
         fine_dev_ = *fine;
@@ -543,52 +491,9 @@ AmgPrecond::AmgPrecond(const HCsr &A, const AmgParams &p, hipStream_t s, const P
         d.use_fine = fine_;
         if (fine_) d.fine = *fine;
         d.build(im_->host, s);
-        if (fine_) fine_dev_.dinv32 = d.fine.dinv32;
     };
     if (p.refreshable && !fine_ && !p.fused_restriction && im_->host.size() >= 2) refresh_setup(im_->rf, im_->host, s);
-    if (p.precision == 32 && fine_) {
-        // The FP32 V-cycle loses the weakly pinned constant mode of the Poisson operator
-        // (A = A0 + E with A0 1 = 0 and E nonzero only at the pinned cells), and BiCGSTAB
-        // then needs several times the iterations. The cell areas w make W A0 symmetric, so
-        // w^T A0 = 0 and w^T A = (w o a)^T with a = A 1 nonzero only at the pins. Writing
-        // r = r' + c a with c = w^T r / w^T a gives A^-1 r = A^-1 r' + c 1, where r' has no
-        // component along the constant mode; the V-cycle sees r' and c 1 is added in FP64.
-        auto &d = im_->d32;
-        const HCsr &H = A;
-        auto rowsum = [&](int i) {
-            double acc = 0;
-            for (int k = H.rp[i]; k < H.rp[i + 1]; k++) acc += H.v[k];
-            return acc;
-        };
-        const int nx = fine->nx, cc = fine->centre;
-        auto area = [&](int ip) {
-            double dx = 0, dy = 0;
-            CUIBM_HIP(hipMemcpy(&dx, fine->dx + ip % nx, sizeof(double), hipMemcpyDeviceToHost));
-            CUIBM_HIP(hipMemcpy(&dy, fine->dy + ip / nx, sizeof(double), hipMemcpyDeviceToHost));
-            return dx * dy;
-        };
-        if (!fine->dx || !fine->dy) throw Error("deflation needs the cell widths of the stencil operator", ERR_ARGUMENT);
-        CUIBM_HIP(hipStreamSynchronize(s));
-        const double a0 = rowsum(0), ac = cc > 0 ? rowsum(cc) : 0.0;
-        const double wa = area(0) * a0 + (cc > 0 ? area(cc) * ac : 0.0);
-        if (!(wa > 0)) throw Error("the Poisson operator has no pinned cell to deflate", ERR_ARGUMENT);
-        d.defl_part.alloc(RED_GRID);
-        d.defl_c.alloc(1);
-        launch_fill(d.defl_c.p(), 0.0, 1, s);
-        d.inv_wa = 1.0 / wa;
-        P5Dev f = *fine;
-        f.defl = d.defl_c.p();
-        f.defl_a0 = a0;
-        f.defl_ac = ac;
-        f.defl_part = d.defl_part.p();
-        f.defl_inv_wa = d.inv_wa;
-        d.probe = &im_->probe;
-        d.prm = p;
-        d.use_fine = true;
-        d.fine = f;
-        d.build(im_->host, s);
-        fine_dev_ = d.fine;
-    } else if (p.precision == 32) setup(im_->d32);
+    if (p.precision == 32) setup(im_->d32);
     else if (p.precision == 3264) setup(im_->d3264);
     else setup(im_->d64);
     // keep only the sizes of the host hierarchy
@@ -600,12 +505,20 @@ AmgPrecond::AmgPrecond(const HCsr &A, const AmgParams &p, hipStream_t s, const P
     }
 }
 
-AmgPrecond::~AmgPrecond() = default;
+AmgPrecond::AmgPrecond(const std::vector<double> &dx, const std::vector<double> &dy, double dt, const P5Dev &fine,
+                       const AmgParams &p, hipStream_t s)
+    : im_(new Impl), prm_(p), fine_(true), fine_dev_(fine) {
+    check_precision(p.precision);
+    if ((int)dx.size() != fine.nx || (int)dy.size() != fine.ny)
+        throw Error("stencil and grid sizes differ", ERR_ARGUMENT);
+    im_->mg.reset(new TensorMg(dx, dy, dt, fine.centre, p.precision, p.coarse_max, fine.dx, fine.dy, s));
+}
 
-double AmgPrecond::deflation_inv_wa() const { return fine_dev_.defl ? im_->d32.inv_wa : 0.0; }
+AmgPrecond::~AmgPrecond() = default;
 
 void AmgPrecond::set_stop(const double *stop) {
     stop_ = stop;
+    if (im_->mg) im_->mg->set_stop(stop);
     im_->each([&](auto &d) {
         d.stop = stop;
         d.fine.stop = stop;
@@ -613,23 +526,16 @@ void AmgPrecond::set_stop(const double *stop) {
 }
 
 void AmgPrecond::apply(const double *r, double *z, hipStream_t s) {
-    if (prm_.precision == 32) im_->d32.apply(r, z, s);
+    if (im_->mg) im_->mg->apply(r, z, s, false);
+    else if (prm_.precision == 32) im_->d32.apply(r, z, s);
     else if (prm_.precision == 3264) im_->d3264.apply(r, z, s);
     else im_->d64.apply(r, z, s);
 }
 
-InputWeights AmgPrecond::input_weights() const {
-    InputWeights w;
-    if (!fine_dev_.defl) return w;
-    w.wx = fine_dev_.dx;
-    w.wy = fine_dev_.dy;
-    w.nx = fine_dev_.nx;
-    w.part = im_->d32.defl_part.p();
-    return w;
-}
+InputWeights AmgPrecond::input_weights() const { return im_->mg ? im_->mg->weights() : InputWeights{}; }
 
 void AmgPrecond::apply_weighted(const double *r, double *z, hipStream_t s) {
-    if (fine_dev_.defl) im_->d32.apply(r, z, s, true);
+    if (im_->mg) im_->mg->apply(r, z, s, true);
     else apply(r, z, s);
 }
 
@@ -652,47 +558,45 @@ static double value_bytes(int precision) { return precision == 64 ? 8.0 : 4.0; }
 static double vector_bytes(int precision) { return precision == 32 ? 4.0 : 8.0; }
 
 double AmgPrecond::level0_sweep_bytes() const {
+    if (fine_)  // x, b, xn, coefficient arrays
+        return (double)fine_dev_.nx * fine_dev_.ny * (8 + 8 + 8) + 32.0 * (fine_dev_.nx + fine_dev_.ny);
     const double sv = value_bytes(prm_.precision);
     const auto &A = im_->host[0].A;
     const double n = A.n, nnz = (double)A.ci.size();
-    if (fine_) return n * (8 + 8 + 8) + 32.0 * (fine_dev_.nx + fine_dev_.ny);  // x, b, xn, coefficient arrays
     return nnz * (sv + 4) + 4 * (n + 1) + n * (8 + 8 + 8 + sv);  // A, rowptr, x, b, xn, dinv
 }
 
 void AmgPrecond::level0_pre(const double *b, double *x2, double *r, hipStream_t s) {
     if (!fine_) throw Error("the finest AMG level is not in stencil form", ERR_ARGUMENT);
-    if (prm_.precision == 32)  // FP32 level vectors in the caller's (larger) buffers
-        launch_p5_pre(fine_dev_, (float)prm_.omega, b, reinterpret_cast<float *>(x2), reinterpret_cast<float *>(r),
-                      s);
-    else
-        launch_p5_pre(fine_dev_, prm_.omega, b, x2, r, s);
+    if (im_->mg) im_->mg->fine_first(b, s);
+    else launch_p5_pre(fine_dev_, prm_.omega, b, x2, r, s);
 }
 
 void AmgPrecond::level0_post(double *x2, const double *b, double *x, hipStream_t s) {
     if (!fine_) throw Error("the finest AMG level is not in stencil form", ERR_ARGUMENT);
-    if (prm_.precision == 32) {
-        auto &L = im_->d32.lv[0];
-        float *x2f = reinterpret_cast<float *>(x2);
-        launch_csr_op<float, float, OP_PROLONG>(L.lanesP, L.P, im_->d32.lv[1].x.p(), nullptr, nullptr, x2f, 0.0f, s);
-        launch_p5_sweep2(fine_dev_, (float)prm_.omega, x2f, b, x, s);
-    } else if (prm_.precision == 3264) {
+    if (im_->mg) {
+        im_->mg->fine_last(b, x, s);
+        return;
+    }
+    if (prm_.precision == 3264) {
         auto &L = im_->d3264.lv[0];
         launch_csr_op<float, double, OP_PROLONG>(L.lanesP, L.P, im_->d3264.lv[1].x.p(), nullptr, nullptr, x2, 0.0, s);
-        launch_p5_sweep2(fine_dev_, prm_.omega, x2, b, x, s);
     } else {
         auto &L = im_->d64.lv[0];
         launch_csr_op<double, double, OP_PROLONG>(L.lanesP, L.P, im_->d64.lv[1].x.p(), nullptr, nullptr, x2, 0.0, s);
-        launch_p5_sweep2(fine_dev_, prm_.omega, x2, b, x, s);
     }
+    launch_p5_sweep2(fine_dev_, prm_.omega, x2, b, x, s);
 }
 
 double AmgPrecond::level0_pre_bytes() const {
+    if (im_->mg) return im_->mg->fine_first_bytes();
     const double sx = vector_bytes(prm_.precision);
     // b (the FP64 Krylov vector) and D^-1 in; x2, r out
     return (8.0 + 3 * sx) * im_->host[0].A.n + 32.0 * (fine_dev_.nx + fine_dev_.ny);
 }
 
 double AmgPrecond::level0_post_bytes() const {
+    if (im_->mg) return im_->mg->fine_last_bytes();
     const double sv = value_bytes(prm_.precision), sx = vector_bytes(prm_.precision);
     const double n = im_->host[0].A.n, nc = im_->host[1].A.n, nnzP = (double)im_->host[0].P.ci.size();
     const double prolong = nnzP * (sv + 4) + 4 * (n + 1) + nc * sx + 2 * n * sx;  // P, xc; x2 read-modify-write
@@ -703,6 +607,15 @@ double AmgPrecond::level0_post_bytes() const {
 
 AmgHierarchyInfo AmgPrecond::info() const {
     AmgHierarchyInfo I;
+    if (im_->mg) {  // five-point rows, implicit interpolation
+        for (const auto &g : im_->mg->sizes()) {
+            I.n.push_back(g.first * g.second);
+            I.nnz.push_back(5 * g.first * g.second - 2 * (g.first + g.second));
+            I.nnzP.push_back(0);
+        }
+        I.levels = (int)I.n.size();
+        return I;
+    }
     I.levels = (int)im_->host.size();
     for (auto &L : im_->host) {
         I.n.push_back(L.A.n);
@@ -713,6 +626,7 @@ AmgHierarchyInfo AmgPrecond::info() const {
 }
 
 std::vector<double> AmgPrecond::launch_bytes() const {
+    if (im_->mg) return im_->mg->launch_bytes();
     // distinct arrays per kernel; matrix values and D^-1 take sv bytes, level vectors sx:
     // CSR product = nnz*(sv+4) + 4(n+1) + sx ncol (x) + sx n (y)
     const double sv = value_bytes(prm_.precision), sx = vector_bytes(prm_.precision);
@@ -723,8 +637,6 @@ std::vector<double> AmgPrecond::launch_bytes() const {
         const double n = H[l].A.n, nnz = (double)H[l].A.ci.size();
         const double nc = H[l + 1].A.n, nnzP = (double)H[l].P.ci.size();
         if (l == 0 && fine_) {
-            // (with deflation, the Krylov kernels that produce b also form its weighted partial
-            // sums, and the pre-smoothing kernel finishes them: no launch of its own)
             L.push_back(level0_pre_bytes());
             L.push_back(spmv(nc, n, nnzP));                                          // restriction
             L.push_back(nnzP * (sv + 4) + 4 * (n + 1) + nc * sx + 2 * n * sx);        // prolong-add
@@ -1103,7 +1015,7 @@ static void refresh_levels(AmgDev<V, X> &dv, RefreshData &rf, const std::vector<
         CUIBM_LAUNCH_CHECK();
     }
     RefreshLevel &Cl = rf.lv[L - 1];
-    if (dv.nc <= RF_GJ_MAX && !dv.fine.defl) {
+    if (dv.nc <= RF_GJ_MAX) {
         hipLaunchKernelGGL((k_rf_gj<V>), dim3(1), dim3(1024), 0, s, Cl.n, Cl.Arp.p(), Cl.Aci.p(), Cl.Av.p(),
                            dv.coarse_inv.p(), dv.ld, rf.flag.p() + 1);
         CUIBM_LAUNCH_CHECK();
@@ -1118,8 +1030,7 @@ static void refresh_levels(AmgDev<V, X> &dv, RefreshData &rf, const std::vector<
     Ac.v.resize(Ac.ci.size());
     if (!Ac.v.empty()) Cl.Av.download(Ac.v.data(), Ac.v.size(), s);
     CUIBM_HIP(hipStreamSynchronize(s));
-    std::vector<double> inv = dense_inverse(Ac);
-    if (dv.fine.defl) AmgDev<V, X>::deflate_coarse(inv, dv.nc);
+    const std::vector<double> inv = dense_inverse(Ac);
     std::vector<V> invt((size_t)dv.nc * dv.ld, V(0));
     for (int i = 0; i < dv.nc; i++)
         for (int j = 0; j < dv.nc; j++) invt[(size_t)i * dv.ld + j] = (V)inv[(size_t)i * dv.nc + j];
@@ -1216,12 +1127,8 @@ struct BatchDev {
     std::vector<Lvl> lv;  // lv[0]: the finest level (P0, R0 and its two vectors)
     int ncases = 0;
     const BCase *tab = nullptr;
-    BMapDev pmap{}, tiles{};
-    const int *pfirst = nullptr;
+    BMapDev tiles{};
     BMap tilemap;
-    DArray<double> part, inv_wa;
-    double *defl = nullptr;
-    bool deflate = false;
     double omega = 0.8;
     DArray<const double *> cstop;  // each case's Poisson stop code: the CSR levels skip stopped cases
 
@@ -1329,7 +1236,6 @@ struct BatchDev {
         CUIBM_HIP(hipStreamSynchronize(s));
     }
 
-    static void launch_fill_x(float *p, long n, hipStream_t s) { if (n) launch_fill_f(p, 0.0f, n, s); }
     static void launch_fill_x(double *p, long n, hipStream_t s) { if (n) launch_fill(p, 0.0, n, s); }
 
     void vcycle(size_t l, hipStream_t s) {
@@ -1358,10 +1264,6 @@ struct BatchDev {
     void apply(const double *b, double *x, hipStream_t s) {
         Lvl &F = lv[0], &C = lv[1];
         const X w = (X)omega;
-        if (deflate) {
-            launch_b_wdot(tab, pmap, b, part.p(), s);
-            launch_b_wdot_finish(tab, ncases, pfirst, part.p(), inv_wa.p(), defl, s);
-        }
         launch_b_p5_pre(tab, tiles, w, b, F.xt.p(), F.r.p(), s);
         launch_csr_op<V, X, OP_SPMV>(F.lanesR, F.R, F.r.p(), nullptr, nullptr, C.b.p(), X(0), s, nullptr, C.seg.p(),
                                      cstop.p());
@@ -1373,9 +1275,8 @@ struct BatchDev {
 };
 
 struct BatchAmg::Impl {
-    int precision = 64;
-    BatchDev<double, double> d64;
-    BatchDev<float, float> d32;
+    BatchDev<double, double> d64;  // stored hierarchies
+    std::unique_ptr<BatchMg> mg;   // tensor multigrid
 };
 
 BatchAmg::BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long> &offP, const BCase *tab_dev,
@@ -1383,58 +1284,41 @@ BatchAmg::BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long>
     : im_(new Impl) {
     if (amg.empty()) throw Error("batched V-cycle without cases", ERR_ARGUMENT);
     const int prec = amg[0]->precision();
+    std::vector<TensorMg *> mg;
     for (auto *a : amg) {
         if (a->precision() != prec) throw Error("batched V-cycle: cases of different AMG precisions", ERR_ARGUMENT);
         if (!a->has_stencil_level()) throw Error("batched V-cycle: a case without its stencil finest level", ERR_UNSUPPORTED);
+        if (a->tensor()) mg.push_back(a->tensor());
     }
     if (prec != 64 && prec != 32) throw Error("batched V-cycle: AMG precision 64 or 32", ERR_UNSUPPORTED);
-    im_->precision = prec;
+    if (!mg.empty() && mg.size() != amg.size()) throw Error("batched V-cycle: cases of different hierarchies", ERR_ARGUMENT);
+    if (!mg.empty()) {
+        im_->mg.reset(new BatchMg(mg, offP, tab_dev, tab_host, pmap, pfirst, s));
+        return;
+    }
     const int n = (int)amg.size();
     std::vector<long> tcount(n);
     for (int c = 0; c < n; c++) tcount[c] = p5_tiles(tab_host[c].p5.nx, tab_host[c].p5.ny);
-    const bool deflate = tab_host[0].p5.defl != nullptr;
-    std::vector<double> iw(n, 0.0);
-    for (int c = 0; c < n; c++) {
-        if ((tab_host[c].p5.defl != nullptr) != deflate)
-            throw Error("batched V-cycle: deflation on some cases only", ERR_ARGUMENT);
-        iw[c] = amg[c]->deflation_inv_wa();
-    }
     std::vector<const double *> stops(n);
     for (int c = 0; c < n; c++) stops[c] = tab_host[c].p5.stop;
-    auto setup = [&](auto &B, const auto &cd) {
-        B.omega = amg[0]->prm_.omega;
-        B.tab = tab_dev;
-        B.pmap = pmap;
-        B.pfirst = pfirst;
-        B.build(cd, offP, stops, s);
-        B.tilemap.build(tcount, 1, s);
-        B.tiles = B.tilemap.dev();
-        B.deflate = deflate;
-        if (deflate) {
-            B.inv_wa.upload(iw, s);
-            B.part.alloc(std::max(pmap.nblk, 1));
-            B.defl = const_cast<double *>(tab_host[0].p5.defl);  // the batch's array: case c at defl + c
-        }
-    };
-    if (prec == 32) {
-        std::vector<AmgDev<float, float> *> cd;
-        for (auto *a : amg) cd.push_back(&a->im_->d32);
-        setup(im_->d32, cd);
-    } else {
-        std::vector<AmgDev<double, double> *> cd;
-        for (auto *a : amg) cd.push_back(&a->im_->d64);
-        setup(im_->d64, cd);
-    }
+    BatchDev<double, double> &B = im_->d64;
+    B.omega = amg[0]->prm_.omega;
+    B.tab = tab_dev;
+    std::vector<AmgDev<double, double> *> cd;
+    for (auto *a : amg) cd.push_back(&a->im_->d64);
+    B.build(cd, offP, stops, s);
+    B.tilemap.build(tcount, 1, s);
+    B.tiles = B.tilemap.dev();
     CUIBM_HIP(hipStreamSynchronize(s));
 }
 
 BatchAmg::~BatchAmg() = default;
 
 void BatchAmg::apply(const double *r, double *z, hipStream_t s) {
-    if (im_->precision == 32) im_->d32.apply(r, z, s);
+    if (im_->mg) im_->mg->apply(r, z, s);
     else im_->d64.apply(r, z, s);
 }
 
-int BatchAmg::levels() const { return im_->precision == 32 ? (int)im_->d32.lv.size() : (int)im_->d64.lv.size(); }
+int BatchAmg::levels() const { return im_->mg ? im_->mg->levels() : (int)im_->d64.lv.size(); }
 
 }  // namespace cuibm

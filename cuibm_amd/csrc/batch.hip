@@ -104,7 +104,7 @@ struct LockstepBatch::Impl {
     std::vector<long> offUV, offP;
     std::vector<int> offXP;
     long nUV = 0, nP = 0, nXP = 0;
-    DArray<double> u, uhat, uold, p, N, Nold, rhs1, rhs2, ustar, pstar, xp, dinv1, defl;
+    DArray<double> u, uhat, uold, p, N, Nold, rhs1, rhs2, ustar, pstar, xp, dinv1;
     DArray<double> sc;  // 2 scalar blocks per case (velocity, Poisson)
     std::vector<double> host_sc;
     DArray<BCase> tab;
@@ -114,6 +114,7 @@ struct LockstepBatch::Impl {
     DArray<int> solid;
     int nsolid = 0;
     std::unique_ptr<BatchAmg> amg;
+    std::vector<std::unique_ptr<AmgPrecond>> own;  // cases whose solver holds another kind
     // Krylov workspace per operator
     struct Work {
         DArray<double> r, rs, p, Mp, AMp, sv, Ms, AMs, part;
@@ -294,6 +295,17 @@ LockstepBatch::LockstepBatch(const std::vector<NavierStokesSolver *> &cases, hip
         A[k] = amg[B.order[k]];
         B.solver.push_back(L[k]);
     }
+    // one kind of hierarchy for the batch: where some cases have mg.hpp's levels and others (small
+    // FP64 grids) a stored one, the others get levels of their own too
+    const bool tensor = std::any_of(A.begin(), A.end(), [](AmgPrecond *a) { return a->tensor() != nullptr; });
+    for (int c = 0; c < B.nc && tensor; c++) {
+        if (A[c]->tensor()) continue;
+        AmgParams p = A[c]->params();
+        p.coarse_max = 0;
+        const P5Dev fine = static_cast<PoissonStencil *>(L[c]->op2.get())->dev();
+        B.own.emplace_back(new AmgPrecond(L[c]->dom->dx, L[c]->dom->dy, L[c]->dt, fine, p, s));
+        A[c] = B.own.back().get();
+    }
     // segments
     for (int c = 0; c < B.nc; c++) {
         B.offUV.push_back(B.nUV);
@@ -328,15 +340,10 @@ LockstepBatch::LockstepBatch(const std::vector<NavierStokesSolver *> &cases, hip
         seg_copy(B.xp.p() + B.offXP[c], S.bc[XPLUS].p(), 2 * S.ny - 1, s);
         launch_diag_inv(S.LHS1, B.dinv1.p() + B.offUV[c], s);
     }
-    // scalar blocks, deflation constants, the case table
+    // scalar blocks, the case table
     B.sc.alloc((size_t)2 * B.nc * SC_COUNT);
     launch_fill(B.sc.p(), 0.0, 2 * B.nc * SC_COUNT, s);
     B.host_sc.assign((size_t)2 * B.nc * SC_COUNT, 0.0);
-    const bool deflate = A[0]->fine_dev().defl != nullptr;
-    if (deflate) {
-        B.defl.alloc(B.nc);
-        launch_fill(B.defl.p(), 0.0, B.nc, s);
-    }
     B.tab_host.resize(B.nc);
     for (int c = 0; c < B.nc; c++) {
         luoIBM &S = *L[c];
@@ -357,10 +364,6 @@ LockstepBatch::LockstepBatch(const std::vector<NavierStokesSolver *> &cases, hip
         C.scP = B.sc.p() + (size_t)(2 * c + 1) * SC_COUNT;
         C.p5 = A[c]->fine_dev();
         C.p5.stop = C.scP + SC_STOP;
-        C.p5.defl = deflate ? B.defl.p() + c : nullptr;
-        C.p5.defl_part = nullptr;  // the batch forms each case's c in k_b_wdot_finish
-        if (deflate != (A[c]->fine_dev().defl != nullptr))
-            throw Error("lockstep batch: the cases' AMG precisions must agree", ERR_ARGUMENT);
         C.fI = S.startI;
         C.fJ = S.startJ;
         C.fncx = S.numCellsX;

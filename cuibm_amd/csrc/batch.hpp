@@ -99,27 +99,40 @@ void launch_b_force(const BCase *tab, int ncases, const double *u, const double 
                     double *out, hipStream_t s);
 
 // ---- batched finest AMG level (k_stencil.hip) ----
-// deflation: partial sums of w_i r_i per block (P map) and, per case, c = sum * inv_wa[c]
+// the constant mode of each case's input: partial sums of w_i r_i per block (P map) and, per case, c = sum * inv_wa[c]
 // into defl[c]
 void launch_b_wdot(const BCase *tab, const BMapDev &m, const double *r, double *part, hipStream_t s);
 void launch_b_wdot_finish(const BCase *tab, int ncases, const int *first, const double *part, const double *inv_wa,
                           double *defl, hipStream_t s);
 // the tile kernels of the finest level per case (tile map: TX x TY tiles per case)
-void launch_b_p5_pre(const BCase *tab, const BMapDev &tiles, float omega, const double *b, float *x2, float *r,
-                     hipStream_t s);
 void launch_b_p5_pre(const BCase *tab, const BMapDev &tiles, double omega, const double *b, double *x2, double *r,
                      hipStream_t s);
-void launch_b_p5_sweep2(const BCase *tab, const BMapDev &tiles, float omega, const float *x, const double *b,
-                        double *xo, hipStream_t s);
 void launch_b_p5_sweep2(const BCase *tab, const BMapDev &tiles, double omega, const double *x, const double *b,
                         double *xo, hipStream_t s);
 // tiles of one case's finest level
 int p5_tiles(int nx, int ny);
 
-// The AMG V-cycles of all cases as one preconditioner: the finest level per case in
-// stencil form (the tile kernels above), the CSR levels concatenated block-diagonally, the
-// dense coarsest solves per case. Built from the cases' own preconditioners, all of one
-// precision (64 or 32); with 32 and a pinned operator the constant mode is deflated per case.
+class TensorMg;
+
+// The multigrid cycles of all cases as one preconditioner (mg.hip): each level of every case
+// that has it is one launch, the constant mode is carried per case.
+class BatchMg {
+  public:
+    BatchMg(const std::vector<TensorMg *> &mg, const std::vector<long> &offP, const BCase *tab_dev,
+            const std::vector<BCase> &tab_host, const BMapDev &pmap, const int *pfirst, hipStream_t s);
+    ~BatchMg();
+    void apply(const double *r, double *z, hipStream_t s);
+    int levels() const;
+
+  private:
+    struct Impl;
+    std::unique_ptr<Impl> im_;
+};
+
+// The cases' own preconditioners as one, all of one precision (64 or 32) and of one kind:
+// mg.hpp's levels (BatchMg), or stored hierarchies: the finest level per case in stencil form
+// (the tile kernels above), the CSR levels concatenated block-diagonally, the dense coarsest
+// solves per case.
 class BatchAmg {
   public:
     BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long> &offP, const BCase *tab_dev,

@@ -142,32 +142,29 @@ __global__ void k_p5_dinv(P5Dev A, double *__restrict__ dinv) {
 }
 
 // the coupling magnitudes of the columns and rows one tile (with a halo of 2) touches,
-// staged in LDS in the compute type T; li, lj below are halo-2 tile coordinates
+// staged in LDS in the compute type double; li, lj below are halo-2 tile coordinates
 // (I = I0 - 2 + li)
-template <class T>
 struct TileCoef {
-    T e[W2], w[W2], n[H2], s[H2];
+    double e[W2], w[W2], n[H2], s[H2];
 };
 
-template <class T>
-__device__ __forceinline__ void load_coef(const P5Dev &A, int I0, int J0, TileCoef<T> &c) {
+__device__ __forceinline__ void load_coef(const P5Dev &A, int I0, int J0, TileCoef &c) {
     for (int k = threadIdx.x; k < W2; k += blockDim.x) {
         const int I = I0 - 2 + k;
         const bool in = I >= 0 && I < A.nx;
-        c.e[k] = in ? (T)A.cE[I] : T(0);
-        c.w[k] = in ? (T)A.cW[I] : T(0);
+        c.e[k] = in ? A.cE[I] : 0.0;
+        c.w[k] = in ? A.cW[I] : 0.0;
     }
     for (int k = threadIdx.x; k < H2; k += blockDim.x) {
         const int J = J0 - 2 + k;
         const bool in = J >= 0 && J < A.ny;
-        c.n[k] = in ? (T)A.cN[J] : T(0);
-        c.s[k] = in ? (T)A.cS[J] : T(0);
+        c.n[k] = in ? A.cN[J] : 0.0;
+        c.s[k] = in ? A.cS[J] : 0.0;
     }
 }
 
-template <class T>
-__device__ __forceinline__ T t_diag(const P5Dev &A, const TileCoef<T> &c, int li, int lj, int I, int J, int ip) {
-    T t = 0;
+__device__ __forceinline__ double t_diag(const P5Dev &A, const TileCoef &c, int li, int lj, int I, int J, int ip) {
+    double t = 0;
     if (I != A.nx - 1) t += c.e[li];
     if (I != 0) t += c.w[li];
     if (J != A.ny - 1) t += c.n[lj];
@@ -177,10 +174,10 @@ __device__ __forceinline__ T t_diag(const P5Dev &A, const TileCoef<T> &c, int li
     return t;
 }
 
-template <class T, class F>
-__device__ __forceinline__ T t_row(const P5Dev &A, const TileCoef<T> &c, int li, int lj, int I, int J, T d, F x,
+template <class F>
+__device__ __forceinline__ double t_row(const P5Dev &A, const TileCoef &c, int li, int lj, int I, int J, double d, F x,
                                    int sy) {
-    T s = 0;
+    double s = 0;
     if (J != 0) s += (-c.s[lj]) * x(-sy);
     if (I != 0) s += (-c.w[li]) * x(-1);
     s += d * x(0);
@@ -189,63 +186,27 @@ __device__ __forceinline__ T t_row(const P5Dev &A, const TileCoef<T> &c, int li,
     return s;
 }
 
-// D^-1 in the compute type: the FP64 array, or its FP32 copy for the FP32 V-cycle
-template <class T>
-__device__ __forceinline__ const T *dinv_of(const P5Dev &A);
-template <>
-__device__ __forceinline__ const double *dinv_of<double>(const P5Dev &A) { return A.dinv; }
-template <>
-__device__ __forceinline__ const float *dinv_of<float>(const P5Dev &A) { return A.dinv32; }
-
 constexpr int N2 = H2 * W2, N1 = H1 * W1, R2 = (N2 + 255) / 256, R1 = (N1 + 255) / 256;
 
-// pre-smoothing (two sweeps from x = 0) and residual on one tile, in the compute type T
-// (b is the FP64 Krylov vector; x2 and r are level vectors of type T); all global loads
-// of a thread are issued before the first is used
-template <class T>
-__device__ __forceinline__ void p5_pre_tile(const P5Dev &A, T w, const double *__restrict__ b, T *__restrict__ x2g,
-                                            T *__restrict__ rg, int tiles_x, int t) {
+// pre-smoothing (two sweeps from x = 0) and residual on one tile; all global loads of a thread
+// are issued before the first is used
+__device__ __forceinline__ void p5_pre_tile(const P5Dev &A, double w, const double *__restrict__ b, double *__restrict__ x2g,
+                                            double *__restrict__ rg, int tiles_x, int t) {
     const double stopv = A.stop ? *A.stop : 0.0;  // the Krylov solve's stop code, tested after the loads
-    __shared__ TileCoef<T> cf;
-    __shared__ T sb[N2], swd[N2], sx2[N1];
+    __shared__ TileCoef cf;
+    __shared__ double sb[N2], swd[N2], sx2[N1];
     const int I0 = (t % tiles_x) * TX, J0 = (t / tiles_x) * TY;
     load_coef(A, I0, J0, cf);
-    const T *dinv = dinv_of<T>(A);
-    // the deflation constant c, wanted only where a pin lies in the tile or its halo
-    double cdefl = 0.0;
-    if (A.defl) {
-        auto near = [&](int ip) {
-            const int I = ip % A.nx, J = ip / A.nx;
-            return I >= I0 - 2 && I < I0 + TX + 2 && J >= J0 - 2 && J < J0 + TY + 2;
-        };
-        if (near(0) || (A.centre > 0 && near(A.centre))) {
-            if (A.defl_part) {  // uniform per block: the partials in a fixed order, as one finish block would
-                __shared__ double cs;
-                double acc[1] = {0};
-                for (int k = threadIdx.x; k < RED_GRID; k += 256) acc[0] += A.defl_part[k];
-                block_sum<1>(acc);
-                if (threadIdx.x == 0) {
-                    cs = acc[0] * A.defl_inv_wa;
-                    if (t == 0) A.defl[0] = cs;  // for the post-smoothing kernel
-                }
-                __syncthreads();
-                cdefl = cs;
-            } else {
-                cdefl = A.defl[0];
-            }
-        }
-    }
-    T bv[R2], dv[R2];
+    const double *dinv = A.dinv;
+    double bv[R2], dv[R2];
 #pragma unroll
     for (int m = 0; m < R2; m++) {
         const int k = threadIdx.x + 256 * m;
         const int I = I0 - 2 + k % W2, J = J0 - 2 + k / W2;
         const bool in = k < N2 && inside(A, I, J);
         const int ip = in ? J * A.nx + I : 0;
-        double bb = in ? b[ip] : 0.0;
-        if (A.defl && in && (ip == 0 || ip == A.centre)) bb -= cdefl * (ip == 0 ? A.defl_a0 : A.defl_ac);
-        bv[m] = (T)bb;
-        dv[m] = in ? dinv[ip] : T(0);
+        bv[m] = in ? b[ip] : 0.0;
+        dv[m] = in ? dinv[ip] : 0.0;
     }
     if (stopv != 0.0) return;  // uniform across the block, before the first barrier
 #pragma unroll
@@ -260,11 +221,11 @@ __device__ __forceinline__ void p5_pre_tile(const P5Dev &A, T w, const double *_
     for (int k = threadIdx.x; k < N1; k += blockDim.x) {
         const int li = k % W1 + 1, lj = k / W1 + 1;
         const int I = I0 - 2 + li, J = J0 - 2 + lj;
-        T v = 0;
+        double v = 0;
         if (inside(A, I, J)) {
             const int c = lj * W2 + li;
-            const T d = t_diag(A, cf, li, lj, I, J, J * A.nx + I);
-            const T s = t_row(A, cf, li, lj, I, J, d, [&](int o) { return swd[c + o] * sb[c + o]; }, W2);
+            const double d = t_diag(A, cf, li, lj, I, J, J * A.nx + I);
+            const double s = t_row(A, cf, li, lj, I, J, d, [&](int o) { return swd[c + o] * sb[c + o]; }, W2);
             v = swd[c] * sb[c] + swd[c] * (sb[c] - s);
         }
         sx2[k] = v;
@@ -276,40 +237,37 @@ __device__ __forceinline__ void p5_pre_tile(const P5Dev &A, T w, const double *_
         if (!inside(A, I, J)) continue;
         const int ip = J * A.nx + I;
         const int c1 = (lj + 1) * W1 + li + 1, c2 = (lj + 2) * W2 + li + 2;
-        const T d = t_diag(A, cf, li + 2, lj + 2, I, J, ip);
-        const T s = t_row(A, cf, li + 2, lj + 2, I, J, d, [&](int o) { return sx2[c1 + o]; }, W1);
+        const double d = t_diag(A, cf, li + 2, lj + 2, I, J, ip);
+        const double s = t_row(A, cf, li + 2, lj + 2, I, J, d, [&](int o) { return sx2[c1 + o]; }, W1);
         x2g[ip] = sx2[c1];
         rg[ip] = sb[c2] - s;
     }
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) k_p5_pre(P5Dev A, T w, const double *__restrict__ b, T *__restrict__ x2g,
-                                                T *__restrict__ rg, int tiles_x, int ntiles) {
+__global__ void __launch_bounds__(256) k_p5_pre(P5Dev A, double w, const double *__restrict__ b, double *__restrict__ x2g,
+                                                double *__restrict__ rg, int tiles_x, int ntiles) {
     const int t = xcd_band(ntiles);
     if (t >= ntiles) return;  // uniform per block
-    p5_pre_tile<T>(A, w, b, x2g, rg, tiles_x, t);
+    p5_pre_tile(A, w, b, x2g, rg, tiles_x, t);
 }
 
-// two weighted-Jacobi sweeps on one tile in the compute type T: x (halo 2, a level
-// vector) -> y (halo 1) -> xo (tile, the FP64 Krylov vector); b is the FP64 Krylov vector
-template <class T>
-__device__ __forceinline__ void p5_sweep2_tile(const P5Dev &A, T w, const T *__restrict__ x,
+// two weighted-Jacobi sweeps on one tile: x (halo 2) -> y (halo 1) -> xo (tile)
+__device__ __forceinline__ void p5_sweep2_tile(const P5Dev &A, double w, const double *__restrict__ x,
                                                const double *__restrict__ b, double *__restrict__ xo, int tiles_x,
                                                int t) {
     const double stopv = A.stop ? *A.stop : 0.0;  // the Krylov solve's stop code, tested after the loads
-    __shared__ TileCoef<T> cf;
-    __shared__ T sx[N2], sb[N1], swd[N1];
+    __shared__ TileCoef cf;
+    __shared__ double sx[N2], sb[N1], swd[N1];
     const int I0 = (t % tiles_x) * TX, J0 = (t / tiles_x) * TY;
     load_coef(A, I0, J0, cf);
-    const T *dinv = dinv_of<T>(A);
-    T xv[R2], bv[R1], dv[R1];
+    const double *dinv = A.dinv;
+    double xv[R2], bv[R1], dv[R1];
 #pragma unroll
     for (int m = 0; m < R2; m++) {
         const int k = threadIdx.x + 256 * m;
         const int I = I0 - 2 + k % W2, J = J0 - 2 + k / W2;
         const bool in = k < N2 && inside(A, I, J);
-        xv[m] = in ? x[J * A.nx + I] : T(0);
+        xv[m] = in ? x[J * A.nx + I] : 0.0;
     }
 #pragma unroll
     for (int m = 0; m < R1; m++) {
@@ -317,12 +275,9 @@ __device__ __forceinline__ void p5_sweep2_tile(const P5Dev &A, T w, const T *__r
         const int I = I0 - 1 + k % W1, J = J0 - 1 + k / W1;
         const bool in = k < N1 && inside(A, I, J);
         const int ip = in ? J * A.nx + I : 0;
-        double bb = in ? b[ip] : 0.0;
-        if (A.defl && in && (ip == 0 || ip == A.centre)) bb -= A.defl[0] * (ip == 0 ? A.defl_a0 : A.defl_ac);
-        bv[m] = (T)bb;
-        dv[m] = in ? dinv[ip] : T(0);
+        bv[m] = in ? b[ip] : 0.0;
+        dv[m] = in ? dinv[ip] : 0.0;
     }
-    const double cdefl = A.defl ? A.defl[0] : 0.0;
     if (stopv != 0.0) return;  // uniform across the block, before the first barrier
 #pragma unroll
     for (int m = 0; m < R2; m++) {
@@ -339,25 +294,25 @@ __device__ __forceinline__ void p5_sweep2_tile(const P5Dev &A, T w, const T *__r
     }
     __syncthreads();
     // first sweep on the halo-1 region, kept in registers until every read of sx is done
-    T yv[R1];
+    double yv[R1];
 #pragma unroll
     for (int m = 0; m < R1; m++) {
         const int k = threadIdx.x + 256 * m;
-        T v = 0;
+        double v = 0;
         if (k < N1) {
             const int li = k % W1 + 1, lj = k / W1 + 1;
             const int I = I0 - 2 + li, J = J0 - 2 + lj;
             if (inside(A, I, J)) {
                 const int c = lj * W2 + li;
-                const T d = t_diag(A, cf, li, lj, I, J, J * A.nx + I);
-                const T s = t_row(A, cf, li, lj, I, J, d, [&](int o) { return sx[c + o]; }, W2);
+                const double d = t_diag(A, cf, li, lj, I, J, J * A.nx + I);
+                const double s = t_row(A, cf, li, lj, I, J, d, [&](int o) { return sx[c + o]; }, W2);
                 v = sx[c] + swd[k] * (sb[k] - s);
             }
         }
         yv[m] = v;
     }
     __syncthreads();
-    T *sy = sx;  // reuse: the halo-1 iterate in halo-1 layout
+    double *sy = sx;  // reuse: the halo-1 iterate in halo-1 layout
 #pragma unroll
     for (int m = 0; m < R1; m++) {
         const int k = threadIdx.x + 256 * m;
@@ -370,19 +325,18 @@ __device__ __forceinline__ void p5_sweep2_tile(const P5Dev &A, T w, const T *__r
         if (!inside(A, I, J)) continue;
         const int ip = J * A.nx + I;
         const int c1 = (lj + 1) * W1 + li + 1;
-        const T d = t_diag(A, cf, li + 2, lj + 2, I, J, ip);
-        const T s = t_row(A, cf, li + 2, lj + 2, I, J, d, [&](int o) { return sy[c1 + o]; }, W1);
-        xo[ip] = (double)(sy[c1] + swd[c1] * (sb[c1] - s)) + cdefl;
+        const double d = t_diag(A, cf, li + 2, lj + 2, I, J, ip);
+        const double s = t_row(A, cf, li + 2, lj + 2, I, J, d, [&](int o) { return sy[c1 + o]; }, W1);
+        xo[ip] = sy[c1] + swd[c1] * (sb[c1] - s);
     }
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) k_p5_sweep2(P5Dev A, T w, const T *__restrict__ x,
+__global__ void __launch_bounds__(256) k_p5_sweep2(P5Dev A, double w, const double *__restrict__ x,
                                                    const double *__restrict__ b, double *__restrict__ xo, int tiles_x,
                                                    int ntiles) {
     const int t = xcd_band(ntiles);
     if (t >= ntiles) return;
-    p5_sweep2_tile<T>(A, w, x, b, xo, tiles_x, t);
+    p5_sweep2_tile(A, w, x, b, xo, tiles_x, t);
 }
 
 // partial sums of w_i r_i, w_i = dx[I] dy[J], over a fixed grid of RED_GRID blocks
@@ -600,51 +554,29 @@ static void tiles(const P5Dev &A, int &tx, int &nt) {
     nt = tx * ((A.ny + TY - 1) / TY);
 }
 
-template <class T>
-static void p5_pre(const P5Dev &A, T omega, const double *b, T *x2, T *r, hipStream_t s, KernelProbe *probe) {
+void launch_p5_pre(const P5Dev &A, double omega, const double *b, double *x2, double *r, hipStream_t s,
+                   KernelProbe *probe) {
     int tx, nt;
     tiles(A, tx, nt);
     if (probe && probe->enabled()) {
         hipEvent_t e0, e1;
         probe->pair(e0, e1);
-        hipExtLaunchKernelGGL(k_p5_pre<T>, dim3(xcd_grid(nt)), dim3(256), 0, s, e0, e1, 0, A, omega, b, x2, r, tx,
-                              nt);
+        hipExtLaunchKernelGGL(k_p5_pre, dim3(xcd_grid(nt)), dim3(256), 0, s, e0, e1, 0, A, omega, b, x2, r, tx, nt);
     } else {
-        hipLaunchKernelGGL(k_p5_pre<T>, dim3(xcd_grid(nt)), dim3(256), 0, s, A, omega, b, x2, r, tx, nt);
+        hipLaunchKernelGGL(k_p5_pre, dim3(xcd_grid(nt)), dim3(256), 0, s, A, omega, b, x2, r, tx, nt);
     }
     CUIBM_LAUNCH_CHECK();
 }
 
-template <class T>
-static void p5_sweep2(const P5Dev &A, T omega, const T *x, const double *b, double *xo, hipStream_t s) {
+void launch_p5_sweep2(const P5Dev &A, double omega, const double *x, const double *b, double *xo, hipStream_t s) {
     int tx, nt;
     tiles(A, tx, nt);
-    hipLaunchKernelGGL(k_p5_sweep2<T>, dim3(xcd_grid(nt)), dim3(256), 0, s, A, omega, x, b, xo, tx, nt);
+    hipLaunchKernelGGL(k_p5_sweep2, dim3(xcd_grid(nt)), dim3(256), 0, s, A, omega, x, b, xo, tx, nt);
     CUIBM_LAUNCH_CHECK();
 }
 
-void launch_p5_pre(const P5Dev &A, double omega, const double *b, double *x2, double *r, hipStream_t s,
-                   KernelProbe *probe) {
-    p5_pre<double>(A, omega, b, x2, r, s, probe);
-}
-
-void launch_p5_pre(const P5Dev &A, float omega, const double *b, float *x2, float *r, hipStream_t s,
-                   KernelProbe *probe) {
-    if (!A.dinv32) throw Error("FP32 finest-level smoother without its FP32 D^-1", ERR_ARGUMENT);
-    p5_pre<float>(A, omega, b, x2, r, s, probe);
-}
-
-void launch_p5_sweep2(const P5Dev &A, double omega, const double *x, const double *b, double *xo, hipStream_t s) {
-    p5_sweep2<double>(A, omega, x, b, xo, s);
-}
-
-void launch_p5_sweep2(const P5Dev &A, float omega, const float *x, const double *b, double *xo, hipStream_t s) {
-    if (!A.dinv32) throw Error("FP32 finest-level smoother without its FP32 D^-1", ERR_ARGUMENT);
-    p5_sweep2<float>(A, omega, x, b, xo, s);
-}
-
 void launch_p5_wdot(const P5Dev &A, const double *r, double *part, hipStream_t s) {
-    if (!A.dx || !A.dy) throw Error("deflation needs the cell widths of the stencil operator", ERR_ARGUMENT);
+    if (!A.dx || !A.dy) throw Error("the constant mode needs the cell widths of the stencil operator", ERR_ARGUMENT);
     hipLaunchKernelGGL(k_p5_wdot, dim3(RED_GRID), dim3(BS), 0, s, A, r, part);
     CUIBM_LAUNCH_CHECK();
 }
@@ -737,7 +669,7 @@ void launch_b_spmv_dot(int op, const BCase *tab, const BMapDev &m, const double 
     CUIBM_LAUNCH_CHECK();
 }
 
-// deflation of the pinned constant mode per case (the FP32 V-cycle)
+// the constant mode of each case's input
 __global__ void __launch_bounds__(BS) k_b_wdot(const BCase *__restrict__ tab, BMapDev m, const double *__restrict__ r,
                                                double *__restrict__ part) {
     const BCase &C = tab[m.cs[blockIdx.x]];
@@ -773,42 +705,30 @@ void launch_b_wdot_finish(const BCase *tab, int ncases, const int *first, const 
 }
 
 // the finest-level tile kernels, one block per tile of one case
-template <class T>
-__global__ void __launch_bounds__(256) k_b_p5_pre(const BCase *__restrict__ tab, BMapDev m, T w,
-                                                  const double *__restrict__ b, T *__restrict__ x2g,
-                                                  T *__restrict__ rg) {
+__global__ void __launch_bounds__(256) k_b_p5_pre(const BCase *__restrict__ tab, BMapDev m, double w,
+                                                  const double *__restrict__ b, double *__restrict__ x2g,
+                                                  double *__restrict__ rg) {
     const BCase &C = tab[m.cs[blockIdx.x]];
     const P5Dev A = C.p5;
-    p5_pre_tile<T>(A, w, b + C.offP, x2g + C.offP, rg + C.offP, (A.nx + TX - 1) / TX, m.loc[blockIdx.x]);
+    p5_pre_tile(A, w, b + C.offP, x2g + C.offP, rg + C.offP, (A.nx + TX - 1) / TX, m.loc[blockIdx.x]);
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) k_b_p5_sweep2(const BCase *__restrict__ tab, BMapDev m, T w,
-                                                     const T *__restrict__ x, const double *__restrict__ b,
+__global__ void __launch_bounds__(256) k_b_p5_sweep2(const BCase *__restrict__ tab, BMapDev m, double w,
+                                                     const double *__restrict__ x, const double *__restrict__ b,
                                                      double *__restrict__ xo) {
     const BCase &C = tab[m.cs[blockIdx.x]];
     const P5Dev A = C.p5;
-    p5_sweep2_tile<T>(A, w, x + C.offP, b + C.offP, xo + C.offP, (A.nx + TX - 1) / TX, m.loc[blockIdx.x]);
+    p5_sweep2_tile(A, w, x + C.offP, b + C.offP, xo + C.offP, (A.nx + TX - 1) / TX, m.loc[blockIdx.x]);
 }
 
-void launch_b_p5_pre(const BCase *tab, const BMapDev &tiles, float omega, const double *b, float *x2, float *r,
-                     hipStream_t s) {
-    hipLaunchKernelGGL(k_b_p5_pre<float>, dim3(tiles.nblk), dim3(256), 0, s, tab, tiles, omega, b, x2, r);
-    CUIBM_LAUNCH_CHECK();
-}
 void launch_b_p5_pre(const BCase *tab, const BMapDev &tiles, double omega, const double *b, double *x2, double *r,
                      hipStream_t s) {
-    hipLaunchKernelGGL(k_b_p5_pre<double>, dim3(tiles.nblk), dim3(256), 0, s, tab, tiles, omega, b, x2, r);
-    CUIBM_LAUNCH_CHECK();
-}
-void launch_b_p5_sweep2(const BCase *tab, const BMapDev &tiles, float omega, const float *x, const double *b,
-                        double *xo, hipStream_t s) {
-    hipLaunchKernelGGL(k_b_p5_sweep2<float>, dim3(tiles.nblk), dim3(256), 0, s, tab, tiles, omega, x, b, xo);
+    hipLaunchKernelGGL(k_b_p5_pre, dim3(tiles.nblk), dim3(256), 0, s, tab, tiles, omega, b, x2, r);
     CUIBM_LAUNCH_CHECK();
 }
 void launch_b_p5_sweep2(const BCase *tab, const BMapDev &tiles, double omega, const double *x, const double *b,
                         double *xo, hipStream_t s) {
-    hipLaunchKernelGGL(k_b_p5_sweep2<double>, dim3(tiles.nblk), dim3(256), 0, s, tab, tiles, omega, x, b, xo);
+    hipLaunchKernelGGL(k_b_p5_sweep2, dim3(tiles.nblk), dim3(256), 0, s, tab, tiles, omega, x, b, xo);
     CUIBM_LAUNCH_CHECK();
 }
 

@@ -247,19 +247,10 @@ struct P5Dev {
     const double *cE, *cW, *cN, *cS;   // coupling magnitudes; 0 where the neighbour is missing
     const double *dinv;                // 1 / diagonal, per cell
     const double *stop = nullptr;      // the kernels return at once while *stop != 0
-    const float *dinv32 = nullptr;     // the same in FP32 (V-cycle with FP32 level vectors)
-    const double *dx = nullptr, *dy = nullptr;  // cell widths (the cell areas weight the deflation)
-    // FP64 deflation of the pinned constant mode for the FP32 V-cycle: defl[0] = c, the
-    // input is r - c A 1 (A 1 is a0 at cell 0 and ac at the centre pin) and c is added to
-    // the output. With defl_part, the pre-smoothing kernel forms c itself from those
-    // RED_GRID partial sums of w_i r_i (c = their sum times defl_inv_wa) in the tiles whose
-    // halo holds a pin, and the tile of cell 0 stores it in defl[0] for the post-smoothing
-    // kernel; without, c is read from defl[0]
-    double *defl = nullptr;
-    double defl_a0 = 0, defl_ac = 0;
-    const double *defl_part = nullptr;
-    double defl_inv_wa = 0;
+    const double *dx = nullptr, *dy = nullptr;  // cell widths
 };
+
+class TensorMg;
 
 class AmgPrecond : public Preconditioner {
   public:
@@ -267,9 +258,13 @@ class AmgPrecond : public Preconditioner {
     // fused stencil kernels instead of CSR products with A (the hierarchy below is
     // still built from the CSR A)
     AmgPrecond(const HCsr &A, const AmgParams &p, hipStream_t s, const P5Dev *fine = nullptr);
+    // the operator in stencil form alone, on cells of widths dx, dy: mg.hpp's levels
+    // (p.coarse_max: largest directly solved level, 0 for the size rules there)
+    AmgPrecond(const std::vector<double> &dx, const std::vector<double> &dy, double dt, const P5Dev &fine,
+               const AmgParams &p, hipStream_t s);
     ~AmgPrecond() override;
     void apply(const double *r, double *z, hipStream_t s) override;
-    // the FP32 V-cycle's deflation weights (cell areas) on a stencil finest level
+    // the constant mode's weights (cell areas) of mg.hpp's levels
     InputWeights input_weights() const override;
     void apply_weighted(const double *r, double *z, hipStream_t s) override;
     double restart_reduction() const override {
@@ -293,14 +288,13 @@ class AmgPrecond : public Preconditioner {
     // + residual (b -> x2, r) and prolongation + post-smoothing (x2, b -> x, with the
     // current coarse correction); bytes are their algorithmic bytes
     bool has_stencil_level() const { return fine_; }
+    TensorMg *tensor() const;  // mg.hpp's levels, if those are used
     // events around every finest-level pre-smoothing launch of the live V-cycles
     KernelProbe &pre_probe();
     void level0_pre(const double *b, double *x2, double *r, hipStream_t s);
     void level0_post(double *x2, const double *b, double *x, hipStream_t s);
     double level0_pre_bytes() const;
     double level0_post_bytes() const;
-    // the stencil finest level as the V-cycle sees it (FP32 D^-1, deflation constants),
-    // and 1 / w^T a of the deflation (0 without deflation)
     const P5Dev &fine_dev() const { return fine_dev_; }
     // Numeric set-up on the device for a new matrix whose entries all lie in the pattern
     // the hierarchy was built on (A's own, or its padded superset): A is scattered into
@@ -314,8 +308,8 @@ class AmgPrecond : public Preconditioner {
     // Returns false when an entry of A lies outside the pattern (the caller then builds
     // a new hierarchy). CSR finest level only.
     bool refresh(const DCsr<double> &A, hipStream_t s);
-    double deflation_inv_wa() const;
     int precision() const { return prm_.precision; }
+    const AmgParams &params() const { return prm_; }
 
   private:
     friend class BatchAmg;

@@ -152,10 +152,26 @@ static HCsr download_csr(const DCsr<double> &A, hipStream_t s) {
     return h;
 }
 
+// An operator in stencil form takes the levels of mg.hpp, except where an FP64 solve is held to the
+// FP64 oracle's iterates, which are those of the stored aggregation hierarchy:
+//  - solves to more than MG_RTOL, whose answer beyond the tolerance is the preconditioner's. 336^2
+//    cylinder at 1e-8 (bar 1e-10): u differs from the oracle's by 1.3e-10 after 200 steps and 7e-10
+//    after 400 even where the Poisson solves here are exact, by 2e-15 with the stored hierarchy, at
+//    4.1 ms a step against 1.0. 1024^2 at 1e-9: 7e-11 between hierarchies, 14.7 ms against 1.6;
+//  - up to four times the largest dense level, where p is compared with its weakly pinned constant
+//    (67^2 cylinder at 1e-12: 1.5e-10 against 1e-14).
+// A system of up to coarse_max unknowns is one dense inverse either way.
+constexpr double MG_RTOL = 1e-9;
+static bool tensor_levels(const LinearSolverParams &p, int n, int coarse_max) {
+    if (n <= coarse_max) return false;
+    return p.amgPrecision == 32 || (p.tolerance <= MG_RTOL && n > 4 * coarse_max);
+}
+
+// `fine` and `dom`, when given: A in stencil form and its grid
 static std::unique_ptr<Preconditioner> make_precond(const LinearSolverParams &p, const DCsr<double> &A, hipStream_t s,
-                                                    const P5Dev *fine = nullptr, bool scale0 = false,
-                                                    int coarse_max = 2500, bool fused_restriction = true,
-                                                    int pad_nx = 0) {
+                                                    const P5Dev *fine = nullptr, const Domain *dom = nullptr,
+                                                    double dt = 0, bool scale0 = false, int coarse_max = 2500,
+                                                    bool fused_restriction = true, int pad_nx = 0) {
     switch (p.preconditioner) {
         case NONE: return std::unique_ptr<Preconditioner>(new IdentityPrecond(A.n));
         case DIAGONAL: return std::unique_ptr<Preconditioner>(new JacobiPrecond(A, s));
@@ -168,6 +184,10 @@ static std::unique_ptr<Preconditioner> make_precond(const LinearSolverParams &p,
             ap.refreshable = !fused_restriction;  // rebuilt every step: keep the symbolic structure
             ap.pad_nx = ap.refreshable ? pad_nx : 0;
             ap.restart = p.restartReduction;
+            if (fine && tensor_levels(p, A.n, coarse_max)) {
+                ap.coarse_max = p.amgCoarseMax;
+                return std::unique_ptr<Preconditioner>(new AmgPrecond(dom->dx, dom->dy, dt, *fine, ap, s));
+            }
             return std::unique_ptr<Preconditioner>(new AmgPrecond(download_csr(A, s), ap, s, fine));
         }
         default: throw Error("preconditioner AINV is not supported", ERR_UNSUPPORTED);
@@ -188,7 +208,7 @@ void NavierStokesSolver::buildPreconditioners() {
         op2.reset(new CsrOp(LHS2));
     }
     PC1 = make_precond(db->velocitySolve, LHS1, stream_);
-    PC2 = make_precond(db->PoissonSolve, LHS2, stream_, stencilLHS2() ? &fine : nullptr, mixedScaleLHS2(),
+    PC2 = make_precond(db->PoissonSolve, LHS2, stream_, stencilLHS2() ? &fine : nullptr, dom, dt, mixedScaleLHS2(),
                        amgCoarseMax(), !amgRebuiltEachStep(), amgRebuiltEachStep() ? nx : 0);
     ks1.reset(new Bicgstab(numUV));
     ks2.reset(new Bicgstab(numP));
@@ -564,6 +584,7 @@ int NavierStokesSolver::timeKernel(const std::string &k, int reps, double *ms, d
     else if (k == "vc_pre") b = amg2()->level0_pre_bytes();
     else if (k == "vc_post") b = amg2()->level0_post_bytes();
     if (k == "vc_post") launch_copy(t2.p(), pressure.p(), numP, s);
+    if (k == "vc_post" || k == "vc_pre") PC2->apply(rhs2.p(), t1.p(), s);  // live level vectors
     once();  // warm-up
     hipEvent_t a, e;
     CUIBM_HIP(hipEventCreate(&a));

@@ -10,7 +10,8 @@
 // row order S, W, C, E, N with the same expressions as the assembled matrix, so
 // y = A x is bit-identical to the CSR product.
 //
-// The V-cycle's finest level runs on this form with two fused LDS-tiled kernels
+// The multigrid of mg.hpp runs on this form on every level. The finest level of a stored
+// hierarchy (amg.hip) does with two fused LDS-tiled kernels
 // (pre-smoothing + residual; both post-smoothing sweeps after a row-parallel
 // prolongation) instead of six CSR launches; each block owns a 64 x 16 tile of cells
 // and computes the intermediate iterates on a halo, so the kernels read b (and x)
@@ -88,14 +89,8 @@ class VelocityStencil : public LinOp {
 void launch_p5_pre(const P5Dev &A, double omega, const double *b, double *x2, double *r, hipStream_t s,
                    KernelProbe *probe = nullptr);
 void launch_p5_sweep2(const P5Dev &A, double omega, const double *x, const double *b, double *xo, hipStream_t s);
-// the same in FP32 (the V-cycle with FP32 level vectors): b is the FP64 Krylov vector,
-// x2 and r are FP32 level vectors, the result xo is written as FP64; D^-1 is A.dinv32
-void launch_p5_pre(const P5Dev &A, float omega, const double *b, float *x2, float *r, hipStream_t s,
-                   KernelProbe *probe = nullptr);
-void launch_p5_sweep2(const P5Dev &A, float omega, const float *x, const double *b, double *xo, hipStream_t s);
-// partial sums of w_i r_i (w = cell areas) over RED_GRID blocks, for the deflation
-// constant that the pre-smoothing kernel forms (P5Dev::defl_part); returns at once while
-// the Krylov solve's stop code is set
+// partial sums of w_i r_i (w = cell areas) over RED_GRID blocks, for the constant mode of a
+// multigrid input (mg.hpp); returns at once while the Krylov solve's stop code is set
 void launch_p5_wdot(const P5Dev &A, const double *r, double *part, hipStream_t s);
 // one sweep xn = x + omega D^-1 (b - A x) (timing of the finest-level smoother)
 void launch_p5_sweep(const P5Dev &A, double omega, const double *x, const double *b, double *xn, hipStream_t s);

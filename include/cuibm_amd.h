@@ -47,9 +47,11 @@ const char *cuibm_last_error(void);
  * read <case_folder>/{simParams,flow,domain,bodies}.yaml, apply the command-line
  * overrides in argv (-nu -uPerturb -vPerturb -scaleCV -nsave -nt -dt -velocityTol
  * -poissonTol, plus -amgPrecision 64|32|3264 (as cuibm_bicgstab's amg_precision; in a
- * solver whose Poisson operator has its stencil form, 32 also removes the pinned constant
+ * solver whose Poisson operator has its stencil form, 32 also carries the pinned constant
  * mode in FP64 around the FP32 V-cycle), -amgCoarseMax N (largest coarsest AMG level, solved
- * with a dense inverse: 16..6144, default 2500; 60 for a moving embedded body),
+ * directly: 16..6144, default 2500; 60 for a moving embedded body; a stencil-form operator
+ * with FP32 levels or a tolerance of 1e-9 or less has levels that follow the cell widths, the
+ * coarsest of up to 224 cells an axis unless N says otherwise),
  * -amgRefresh 0|1 (a moving embedded body's Poisson hierarchy is built on a pattern padded
  * around the body's rows and, while each new matrix keeps to it, set up again numerically
  * on the device with its aggregates kept: 1, the default; or built anew on the host every
