@@ -1,37 +1,16 @@
 // Vector, reduction and sparse-product kernels for the Krylov and AMG solvers.
 //
-// Reductions are deterministic: a fixed grid of RED_GRID blocks strides over the
+// Reductions are deterministic: a grid that depends on n alone (red_blocks) strides over the
 // vector, each block reduces its threads in a fixed tree (wavefront shuffles, then
-// LDS across the 4 wavefronts of a 256-thread block) and writes one partial; a
-// single-block kernel then sums the partials in a fixed order. The result depends
-// only on n, never on scheduling.
+// LDS across the 4 wavefronts of a 256-thread block) and writes one partial; the
+// consumer, or a single-block kernel, then sums the partials in a fixed order. The result
+// depends only on n, never on scheduling.
 #include "batch.hpp"
 #include "krylov.hpp"
+#include "krylov_dev.hpp"
 #include "kernels.hpp"
 
 namespace cuibm {
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    return v;
-}
-
-// reduce `k` values per thread across a 256-thread block; thread 0 gets the sums
-template <int K>
-__device__ __forceinline__ void block_sum(double (&v)[K]) {
-    __shared__ double sh[K][BS / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k < K; k++) v[k] = wave_sum(v[k]);
-    if (lane == 0)
-#pragma unroll
-        for (int k = 0; k < K; k++) sh[k][wid] = v[k];
-    __syncthreads();
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int k = 0; k < K; k++) v[k] = (sh[k][0] + sh[k][1]) + (sh[k][2] + sh[k][3]);
-}
 
 template <class T>
 __global__ void k_fill(T *x, T v, long n) {
@@ -111,27 +90,38 @@ void launch_spmv(const DCsr<V> &A, const X *x, X *y, hipStream_t s) {
 template void launch_spmv<double, double>(const DCsr<double> &, const double *, double *, hipStream_t);
 template void launch_spmv<float, double>(const DCsr<float> &, const double *, double *, hipStream_t);
 
-// y = A x with block partials of (y . a) and, when b2 is set, (y . y)
+// y = A x with block partials of (y . a) and, when want_yy is set, (y . y). JAC: x = D^-1 p, formed
+// at every gather, and written to Mp.
+// Each block takes a contiguous chunk of rows, and the chunks of one XCD are contiguous too, so
+// that the gathers of x from neighbouring rows stay in that XCD's L2.
+template <bool JAC>
 __global__ void __launch_bounds__(BS) k_spmv_dot(int n, const int *__restrict__ rp, const int *__restrict__ ci,
                                                  const double *__restrict__ v, const double *__restrict__ x,
+                                                 const double *__restrict__ dinv, double *__restrict__ Mp,
                                                  double *__restrict__ y, const double *__restrict__ a, int want_yy,
-                                                 double *__restrict__ part, const double *__restrict__ stop) {
+                                                 FinArgs f, double *__restrict__ part, const double *__restrict__ stop) {
     const double stopv = stop ? *stop : 0.0;  // read at once, tested after the first row
+    if (JAC && f.part) {
+        double tot[2] = {0, 0};
+        finish_sums<1>(f, tot);
+        if (stopv != 0.0) return;  // uniform, as every return before the last barrier
+        if (fin_ss(tot, f.sc, blockIdx.x == 0 && threadIdx.x == 0) != 0.0) return;
+    }
     double acc[2] = {0, 0};
     bool tested = false;
-    // The first nb blocks (a multiple of 8, so spread evenly over the XCDs) each take a
-    // contiguous chunk of rows, and the chunks of one XCD are contiguous too, so that the
-    // gathers of x from neighbouring rows stay in that XCD's L2; the other blocks write
-    // zero partials.
-    const int nb = min(RED_GRID, (int)((n / BS + 8) / 8 * 8));
-    const int chunk = (n + nb - 1) / nb;
-    const int r0 = (int)blockIdx.x < nb ? xcd_block(nb) * chunk : n, r1 = min(n, r0 + chunk);
+    const int nb = gridDim.x, chunk = (n + nb - 1) / nb, r0 = xcd_block(nb) * chunk, r1 = min(n, r0 + chunk);
     for (int i = r0 + threadIdx.x; i < r1; i += BS) {
-        const double yi = row_dot(rp, ci, v, x, i);
+        double yi;
+        if (JAC) {
+            yi = csr_lane_sum<double, 1>(ci, v, rp[i], rp[i + 1], [&](int c) { return dinv[c] * x[c]; });
+        } else {
+            yi = row_dot(rp, ci, v, x, i);
+        }
         if (!tested) {
             if (stopv != 0.0) return;  // every thread returns here or below: no barrier is reached
             tested = true;
         }
+        if (JAC) Mp[i] = dinv[i] * x[i];
         y[i] = yi;
         acc[0] += yi * a[i];
         acc[1] += yi * yi;
@@ -146,8 +136,16 @@ __global__ void __launch_bounds__(BS) k_spmv_dot(int n, const int *__restrict__ 
 
 void launch_spmv_dot(const DCsr<double> &A, const double *x, double *y, const double *a, bool want_yy, double *part,
                      hipStream_t s, const double *stop) {
-    hipLaunchKernelGGL(k_spmv_dot, dim3(RED_GRID), dim3(BS), 0, s, A.n, A.rp.p(), A.ci.p(), A.v.p(), x, y, a,
-                       (int)want_yy, part, stop);
+    hipLaunchKernelGGL(k_spmv_dot<false>, dim3(red_blocks(A.n)), dim3(BS), 0, s, A.n, A.rp.p(), A.ci.p(), A.v.p(), x,
+                       nullptr, nullptr, y, a, (int)want_yy, FinArgs{}, part, stop);
+    CUIBM_LAUNCH_CHECK();
+}
+
+void launch_spmv_dot_jacobi(const DCsr<double> &A, const double *dinv, const double *p, double *Mp, double *y,
+                            const double *a, bool want_yy, const FinArgs &f, double *part, hipStream_t s,
+                            const double *stop) {
+    hipLaunchKernelGGL(k_spmv_dot<true>, dim3(red_blocks(A.n)), dim3(BS), 0, s, A.n, A.rp.p(), A.ci.p(), A.v.p(), p,
+                       dinv, Mp, y, a, (int)want_yy, f, part, stop);
     CUIBM_LAUNCH_CHECK();
 }
 
@@ -176,7 +174,7 @@ __global__ void __launch_bounds__(BS) k_bicg_init(int n, const int *__restrict__
 
 void launch_bicg_init(const DCsr<double> &A, const double *x, const double *b, double *r, double *p, double *rs,
                       double *part, hipStream_t s) {
-    hipLaunchKernelGGL(k_bicg_init, dim3(RED_GRID), dim3(BS), 0, s, A.n, A.rp.p(), A.ci.p(), A.v.p(), x, b, r, p, rs,
+    hipLaunchKernelGGL(k_bicg_init, dim3(red_blocks(A.n)), dim3(BS), 0, s, A.n, A.rp.p(), A.ci.p(), A.v.p(), x, b, r, p, rs,
                        part);
     CUIBM_LAUNCH_CHECK();
 }
@@ -184,22 +182,33 @@ void launch_bicg_init(const DCsr<double> &A, const double *x, const double *b, d
 // s = r - alpha AMp with partials of (s.s)
 template <bool W>
 __global__ void __launch_bounds__(BS) k_bicg_s(int n, const double *__restrict__ r, const double *__restrict__ AMp,
-                                               double *__restrict__ s, const double *__restrict__ sc,
-                                               double *__restrict__ part, InputWeights w) {
-    const double stopv = sc[SC_STOP], alpha = sc[SC_ALPHA];
+                                               double *__restrict__ s, FinArgs f, double *__restrict__ part,
+                                               InputWeights w) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    double rv = i < n ? r[i] : 0.0, av = i < n ? AMp[i] : 0.0;  // in flight during the finish
+    const double stopv = f.sc[sc_stop(f.par)];
+    double alpha;
+    if (f.part) {
+        double tot[2] = {0, 0};
+        finish_sums<1>(f, tot);
+        if (stopv != 0.0) return;  // uniform, as every return before the last barrier
+        alpha = fin_alpha(tot, f.sc, f.par, blockIdx.x == 0 && threadIdx.x == 0);
+    } else {
+        alpha = f.sc[SC_ALPHA];
+    }
+    if (stopv != 0.0) return;
     double acc[2] = {0, 0};
-    bool tested = false;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double si = r[i] - alpha * AMp[i];
-        if (!tested) {
-            if (stopv != 0.0) return;  // every thread returns here or below: no barrier is reached
-            tested = true;
-        }
+    while (i < n) {
+        const double si = rv - alpha * av;
         s[i] = si;
         acc[0] += si * si;
         if (W) acc[1] += (w.wx[i % w.nx] * w.wy[i / w.nx]) * si;
+        i += gridDim.x * blockDim.x;
+        if (i < n) {
+            rv = r[i];
+            av = AMp[i];
+        }
     }
-    if (stopv != 0.0) return;
     block_sum<2>(acc);
     if (threadIdx.x == 0) {
         part[blockIdx.x] = acc[0];
@@ -207,43 +216,59 @@ __global__ void __launch_bounds__(BS) k_bicg_s(int n, const double *__restrict__
     }
 }
 
-void launch_bicg_s(int n, const double *r, const double *AMp, double *s_, const double *sc, double *part,
+void launch_bicg_s(int n, const double *r, const double *AMp, double *s_, const FinArgs &f, double *part,
                    hipStream_t s, const InputWeights *w) {
-    if (w) hipLaunchKernelGGL(k_bicg_s<true>, dim3(RED_GRID), dim3(BS), 0, s, n, r, AMp, s_, sc, part, *w);
-    else hipLaunchKernelGGL(k_bicg_s<false>, dim3(RED_GRID), dim3(BS), 0, s, n, r, AMp, s_, sc, part, InputWeights{});
+    const dim3 g(red_blocks(n));
+    if (w) hipLaunchKernelGGL(k_bicg_s<true>, g, dim3(BS), 0, s, n, r, AMp, s_, f, part, *w);
+    else hipLaunchKernelGGL(k_bicg_s<false>, g, dim3(BS), 0, s, n, r, AMp, s_, f, part, InputWeights{});
     CUIBM_LAUNCH_CHECK();
 }
 
 // x += alpha Mp + omega Ms; r = s - omega AMs; partials of (rs.r) and (r.r). In the
-// iteration that ended at its half step (SC_STOP = STOP_HALF_PENDING) it applies the
-// half-step update x += alpha Mp alone.
+// iteration that ended at its half step (STOP_HALF_PENDING) it applies the half-step update
+// x += alpha Mp alone.
 __global__ void __launch_bounds__(BS) k_bicg_xr(int n, double *__restrict__ x, const double *__restrict__ Mp,
                                                 const double *__restrict__ Ms, double *__restrict__ r,
                                                 const double *__restrict__ s, const double *__restrict__ AMs,
-                                                const double *__restrict__ rs, const double *__restrict__ sc,
-                                                double *__restrict__ part) {
-    const double stopv = sc[SC_STOP], alpha = sc[SC_ALPHA], omega = sc[SC_OMEGA];
-    const bool half = stopv == STOP_HALF_PENDING;
+                                                const double *__restrict__ rs, FinArgs f, double *__restrict__ part) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    auto at = [&](const double *a) { return i < n ? a[i] : 0.0; };
+    double xv = at(x), mp = at(Mp), ms = at(Ms), sv = at(s), am = at(AMs), rv = at(rs);  // in flight during the finish
+    const double stopv = f.sc[sc_stop(f.par)], half_code = f.sc[SC_STOPS], alpha = f.sc[SC_ALPHA];
+    const bool half = stopv == 0.0 && half_code == STOP_HALF_PENDING;
+    const bool stopped = stopv != 0.0 || half_code != 0.0;
+    double omega = 0;
+    if (f.part) {
+        double tot[2] = {0, 0};
+        finish_sums<2>(f, tot);
+        if (!stopped) omega = fin_omega(tot, f.sc, blockIdx.x == 0 && threadIdx.x == 0);
+    } else {
+        omega = f.sc[SC_OMEGA];
+    }
+    if (stopped && !half) return;  // uniform, as every return before the last barrier
     double acc[2] = {0, 0};
-    bool tested = false;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double xh = x[i] + alpha * Mp[i];
-        const double xi = xh + omega * Ms[i];
-        const double ri = s[i] - omega * AMs[i];
-        if (!tested) {
-            if (stopv != 0.0 && !half) return;  // every thread returns here or below: no barrier is reached
-            tested = true;
-        }
+    while (i < n) {
+        const double xh = xv + alpha * mp;
         if (half) {
             x[i] = xh;
-            continue;
+        } else {
+            const double ri = sv - omega * am;
+            x[i] = xh + omega * ms;
+            r[i] = ri;
+            acc[0] += rv * ri;
+            acc[1] += ri * ri;
         }
-        x[i] = xi;
-        r[i] = ri;
-        acc[0] += rs[i] * ri;
-        acc[1] += ri * ri;
+        i += gridDim.x * blockDim.x;
+        if (i < n) {
+            xv = x[i];
+            mp = Mp[i];
+            ms = Ms[i];
+            sv = s[i];
+            am = AMs[i];
+            rv = rs[i];
+        }
     }
-    if (stopv != 0.0) return;  // includes the half-step update
+    if (half) return;
     block_sum<2>(acc);
     if (threadIdx.x == 0) {
         part[blockIdx.x] = acc[0];
@@ -252,51 +277,60 @@ __global__ void __launch_bounds__(BS) k_bicg_xr(int n, double *__restrict__ x, c
 }
 
 void launch_bicg_xr(int n, double *x, const double *Mp, const double *Ms, double *r, const double *s_,
-                    const double *AMs, const double *rs, const double *sc, double *part, hipStream_t s) {
-    hipLaunchKernelGGL(k_bicg_xr, dim3(RED_GRID), dim3(BS), 0, s, n, x, Mp, Ms, r, s_, AMs, rs, sc, part);
+                    const double *AMs, const double *rs, const FinArgs &f, double *part, hipStream_t s) {
+    hipLaunchKernelGGL(k_bicg_xr, dim3(red_blocks(n)), dim3(BS), 0, s, n, x, Mp, Ms, r, s_, AMs, rs, f, part);
     CUIBM_LAUNCH_CHECK();
 }
 
-// p = r + beta p - beta omega AMp
-__global__ void k_bicg_p(int n, double *__restrict__ p, const double *__restrict__ r, const double *__restrict__ AMp,
-                         const double *__restrict__ sc) {
-    const double stopv = sc[SC_STOP], beta = sc[SC_BETA], omega = sc[SC_OMEGA];
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double v = r[i] + beta * p[i] - beta * omega * AMp[i];
-        if (stopv != 0.0) return;
-        p[i] = v;
-    }
-}
-
-// the same with the weighted partial sums of the new p (a fixed grid of RED_GRID blocks)
-__global__ void __launch_bounds__(BS) k_bicg_pw(int n, double *__restrict__ p, const double *__restrict__ r,
-                                                const double *__restrict__ AMp, const double *__restrict__ sc,
-                                                InputWeights w) {
-    const double stopv = sc[SC_STOP], beta = sc[SC_BETA], omega = sc[SC_OMEGA];
-    double acc[1] = {0};
-    bool tested = false;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double v = r[i] + beta * p[i] - beta * omega * AMp[i];
-        if (!tested) {
-            if (stopv != 0.0) return;  // every thread returns here or below: no barrier is reached
-            tested = true;
+// p = r + beta p - beta omega AMp; W: with the weighted partial sums of the new p
+template <bool W>
+__global__ void __launch_bounds__(BS) k_bicg_p(int n, double *__restrict__ p, const double *__restrict__ r,
+                                               const double *__restrict__ AMp, FinArgs f, InputWeights w) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    double pv = i < n ? p[i] : 0.0, rv = i < n ? r[i] : 0.0, av = i < n ? AMp[i] : 0.0;  // in flight during the finish
+    const double omega = f.sc[SC_OMEGA];
+    double beta;
+    if (f.part) {
+        const bool one = blockIdx.x == 0 && threadIdx.x == 0;
+        const bool stopped = f.sc[sc_stop(f.par)] != 0.0 || f.sc[SC_STOPS] != 0.0;
+        double tot[2] = {0, 0};
+        finish_sums<2>(f, tot);
+        if (stopped) {
+            if (one) pass_stop(f.sc, f.par);
+            return;  // uniform, as every return before the last barrier
         }
-        p[i] = v;
-        acc[0] += (w.wx[i % w.nx] * w.wy[i / w.nx]) * v;
+        beta = fin_beta(tot, f.sc, f.par, f.maxit, one);  // a p past the last iteration is not used
+    } else {
+        if (f.sc[sc_stop(f.par ^ 1)] != 0.0) return;
+        beta = f.sc[SC_BETA];
     }
-    if (stopv != 0.0) return;
+    double acc[1] = {0};
+    while (i < n) {
+        const double v = rv + beta * pv - beta * omega * av;
+        p[i] = v;
+        if (W) acc[0] += (w.wx[i % w.nx] * w.wy[i / w.nx]) * v;
+        i += gridDim.x * blockDim.x;
+        if (i < n) {
+            pv = p[i];
+            rv = r[i];
+            av = AMp[i];
+        }
+    }
+    if (!W) return;
     block_sum<1>(acc);
     if (threadIdx.x == 0) w.part[blockIdx.x] = acc[0];
 }
 
-void launch_bicg_p(int n, double *p, const double *r, const double *AMp, const double *sc, hipStream_t s,
+void launch_bicg_p(int n, double *p, const double *r, const double *AMp, const FinArgs &f, hipStream_t s,
                    const InputWeights *w) {
-    if (w) hipLaunchKernelGGL(k_bicg_pw, dim3(RED_GRID), dim3(BS), 0, s, n, p, r, AMp, sc, *w);
-    else hipLaunchKernelGGL(k_bicg_p, dim3(grid_for(n)), dim3(BS), 0, s, n, p, r, AMp, sc);
+    const dim3 g(red_blocks(n));
+    if (w) hipLaunchKernelGGL(k_bicg_p<true>, g, dim3(BS), 0, s, n, p, r, AMp, f, *w);
+    else hipLaunchKernelGGL(k_bicg_p<false>, g, dim3(BS), 0, s, n, p, r, AMp, f, InputWeights{});
     CUIBM_LAUNCH_CHECK();
 }
 
-// the scalar updates and stopping tests of one finish, from the summed partials tot
+// the scalar updates and stopping tests of one finish of a batched case, from the summed
+// partials tot
 __device__ __forceinline__ void finish_update(int op, const double (&tot)[2], double *__restrict__ sc, double tol,
                                               int maxit) {
     switch (op) {
@@ -337,32 +371,32 @@ __device__ __forceinline__ void finish_update(int op, const double (&tot)[2], do
                 sc[SC_STOP] = STOP_MAXIT;
             break;
         }
-        case FIN_DOT2:
-            sc[SC_D0] = tot[0];
-            sc[SC_D1] = tot[1];
-            break;
     }
 }
 
-// sum the partial groups and update the recurrence scalars (one block); FIN_SS and
-// FIN_BETA then apply the host's stopping tests (cusp::monitor on ||s|| and ||r||, the
-// breakdown tests, the iteration limit) and record the outcome in SC_STOP
-__global__ void __launch_bounds__(1024) k_bicg_finish(const double *__restrict__ part, int op, double *__restrict__ sc,
-                                                      double tol, int maxit) {
-    const double stopv = (op != FIN_INIT && op != FIN_DOT2) ? sc[SC_STOP] : 0.0;  // tested after the loads
-    if (op == FIN_BETA && stopv == STOP_HALF_PENDING) {  // the half-step update is done
-        if (threadIdx.x == 0) sc[SC_STOP] = STOP_HALF;
-        return;
-    }
+// sum the partial groups and update the recurrence scalars (one block)
+__global__ void __launch_bounds__(1024) k_bicg_finish(const double *__restrict__ part, int np, int op, FinArgs f,
+                                                      double rtol) {
+    double *sc = f.sc;
+    const bool start = op == FIN_INIT || op == FIN_RESTART;
+    // the codes that stop this finish, tested after the loads
+    const double stopv = start ? 0.0 : sc[sc_stop(f.par)];
+    const double half = start || op == FIN_ALPHA || op == FIN_SS ? 0.0 : sc[SC_STOPS];
     __shared__ double sh[2][16];
     double v[2] = {0, 0};
     const int ng = (op == FIN_ALPHA || op == FIN_SS) ? 1 : 2;
     for (int g = 0; g < ng; g++) {
         double t = 0;
-        for (int k = threadIdx.x; k < RED_GRID; k += blockDim.x) t += part[g * RED_GRID + k];
+        for (int k = threadIdx.x; k < np; k += blockDim.x) t += part[g * RED_GRID + k];
         v[g] = t;
     }
-    if (stopv != 0.0) return;  // uniform across the block, before the barrier
+    if (stopv != 0.0 || half != 0.0) {  // uniform across the block, before the barrier
+        if (threadIdx.x == 0) {
+            if (op == FIN_SS) sc[SC_STOPS] = stopv;  // what the second half reads
+            if (op == FIN_BETA) pass_stop(sc, f.par);
+        }
+        return;
+    }
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     for (int g = 0; g < ng; g++) {
         double t = wave_sum(v[g]);
@@ -376,31 +410,30 @@ __global__ void __launch_bounds__(1024) k_bicg_finish(const double *__restrict__
         for (int w = 0; w < (int)(blockDim.x >> 6); w++) t += sh[g][w];
         tot[g] = t;
     }
-    finish_update(op, tot, sc, tol, maxit);
-}
-
-void launch_bicg_finish(const double *part, int op, double *sc, hipStream_t s, double tol, int maxit) {
-    hipLaunchKernelGGL(k_bicg_finish, dim3(1), dim3(1024), 0, s, part, op, sc, tol, maxit);
-    CUIBM_LAUNCH_CHECK();
-}
-
-// partial dot products (x.y) and (x.x)
-__global__ void __launch_bounds__(BS) k_dot2(long n, const double *__restrict__ x, const double *__restrict__ y,
-                                             double *__restrict__ part) {
-    double acc[2] = {0, 0};
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        acc[0] += x[i] * y[i];
-        acc[1] += x[i] * x[i];
+    switch (op) {
+        case FIN_INIT:  // (r.r, b.b)
+        case FIN_RESTART:
+            sc[SC_RR] = tot[0];
+            sc[SC_RHO] = tot[0];
+            sc[SC_STOPS] = 0.0;
+            sc[SC_STOP] = 0.0;
+            if (op == FIN_INIT) {
+                sc[SC_BB] = tot[1];
+                sc[SC_D0] = tot[0];
+                sc[SC_ITS] = 0.0;
+                sc[SC_TOL] = rtol * sqrt(tot[1]);
+                if (sqrt(tot[0]) <= sc[SC_TOL]) sc[SC_STOP] = STOP_CONVERGED;
+            }
+            break;
+        case FIN_ALPHA: fin_alpha(tot, sc, f.par, true); break;
+        case FIN_SS: fin_ss(tot, sc, true); break;
+        case FIN_OMEGA: fin_omega(tot, sc, true); break;
+        case FIN_BETA: fin_beta(tot, sc, f.par, f.maxit, true); break;
     }
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = acc[0];
-        part[RED_GRID + blockIdx.x] = acc[1];
-    }
 }
 
-void launch_dot2(long n, const double *x, const double *y, double *part, hipStream_t s) {
-    hipLaunchKernelGGL(k_dot2, dim3(RED_GRID), dim3(BS), 0, s, n, x, y, part);
+void launch_bicg_finish(const double *part, int np, int op, const FinArgs &f, hipStream_t s, double rtol) {
+    hipLaunchKernelGGL(k_bicg_finish, dim3(1), dim3(1024), 0, s, part, np, op, f, rtol);
     CUIBM_LAUNCH_CHECK();
 }
 

@@ -5,6 +5,7 @@
 #include <algorithm>
 
 #include "batch.hpp"
+#include "krylov_dev.hpp"
 #include "stencil.hpp"
 
 namespace cuibm {
@@ -47,27 +48,6 @@ __device__ __forceinline__ double p5_row(const P5Dev &A, int I, int J, double d,
     return s;
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    return v;
-}
-
-template <int K>
-__device__ __forceinline__ void block_sum(double (&v)[K]) {
-    __shared__ double sh[K][BS / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k < K; k++) v[k] = wave_sum(v[k]);
-    if (lane == 0)
-#pragma unroll
-        for (int k = 0; k < K; k++) sh[k][wid] = v[k];
-    __syncthreads();
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int k = 0; k < K; k++) v[k] = (sh[k][0] + sh[k][1]) + (sh[k][2] + sh[k][3]);
-}
-
 // coupling magnitudes, the expressions of LHS2.cu:150-153
 __global__ void k_p5_coef(int nx, int ny, const double *__restrict__ dx, const double *__restrict__ dy, double dt,
                           double *cE, double *cW, double *cN, double *cS) {
@@ -82,21 +62,32 @@ __global__ void k_p5_coef(int nx, int ny, const double *__restrict__ dx, const d
     }
 }
 
-// y = A x with partials of (y . a) and (y . y) over a fixed grid of RED_GRID blocks
-__global__ void __launch_bounds__(BS) k_p5_spmv_dot(P5Dev A, const double *__restrict__ x, double *__restrict__ y,
-                                                    const double *__restrict__ a, int want_yy,
-                                                    double *__restrict__ part) {
+// y = A x with partials of (y . a) and (y . y). JAC: x = D^-1 p, formed at every point of the row,
+// and written to Mp (as the CSR k_spmv_dot).
+template <bool JAC>
+__global__ void __launch_bounds__(BS) k_p5_spmv_dot(P5Dev A, const double *__restrict__ x,
+                                                    const double *__restrict__ dinv, double *__restrict__ Mp,
+                                                    double *__restrict__ y, const double *__restrict__ a, int want_yy,
+                                                    FinArgs f, double *__restrict__ part) {
     const double stopv = A.stop ? *A.stop : 0.0;  // the Krylov solve's stop code, tested after the loads
-    const int n = A.nx * A.ny, blk = xcd_band(RED_GRID);
+    if (JAC && f.part) {
+        double tot[2] = {0, 0};
+        finish_sums<1>(f, tot);
+        if (stopv != 0.0) return;  // uniform, as every return before the last barrier
+        if (fin_ss(tot, f.sc, blockIdx.x == 0 && threadIdx.x == 0) != 0.0) return;
+    }
+    const int n = A.nx * A.ny, nb = gridDim.x, blk = xcd_band(nb);
     double acc[2] = {0, 0};
     bool tested = false;
-    for (int ip = blk * BS + threadIdx.x; ip < n; ip += RED_GRID * BS) {
+    for (int ip = blk * BS + threadIdx.x; ip < n; ip += nb * BS) {
         const int I = ip % A.nx, J = ip / A.nx;
-        const double yi = p5_row(A, I, J, p5_diag(A, I, J, ip), [&](int o) { return x[ip + o]; }, A.nx);
+        const double yi = p5_row(
+            A, I, J, p5_diag(A, I, J, ip), [&](int o) { return JAC ? dinv[ip + o] * x[ip + o] : x[ip + o]; }, A.nx);
         if (!tested) {
             if (stopv != 0.0) return;  // every thread returns here or below: no barrier is reached
             tested = true;
         }
+        if (JAC) Mp[ip] = dinv[ip] * x[ip];
         if (y) y[ip] = yi;
         acc[0] += yi * a[ip];
         acc[1] += yi * yi;
@@ -113,9 +104,9 @@ __global__ void __launch_bounds__(BS) k_p5_spmv_dot(P5Dev A, const double *__res
 __global__ void __launch_bounds__(BS) k_p5_init(P5Dev A, const double *__restrict__ x, const double *__restrict__ b,
                                                 double *__restrict__ r, double *__restrict__ p,
                                                 double *__restrict__ rs, double *__restrict__ part) {
-    const int n = A.nx * A.ny, blk = xcd_band(RED_GRID);
+    const int n = A.nx * A.ny, blk = xcd_band(gridDim.x);
     double acc[2] = {0, 0};
-    for (int ip = blk * BS + threadIdx.x; ip < n; ip += RED_GRID * BS) {
+    for (int ip = blk * BS + threadIdx.x; ip < n; ip += gridDim.x * BS) {
         const int I = ip % A.nx, J = ip / A.nx;
         const double bi = b[ip];
         const double ri = bi - p5_row(A, I, J, p5_diag(A, I, J, ip), [&](int o) { return x[ip + o]; }, A.nx);
@@ -339,13 +330,13 @@ __global__ void __launch_bounds__(256) k_p5_sweep2(P5Dev A, double w, const doub
     p5_sweep2_tile(A, w, x, b, xo, tiles_x, t);
 }
 
-// partial sums of w_i r_i, w_i = dx[I] dy[J], over a fixed grid of RED_GRID blocks
+// partial sums of w_i r_i, w_i = dx[I] dy[J]
 __global__ void __launch_bounds__(BS) k_p5_wdot(P5Dev A, const double *__restrict__ r, double *__restrict__ part) {
     const double stopv = A.stop ? *A.stop : 0.0;
     if (stopv != 0.0) return;
-    const int n = A.nx * A.ny, blk = xcd_band(RED_GRID);
+    const int n = A.nx * A.ny, blk = xcd_band(gridDim.x);
     double acc[1] = {0};
-    for (int ip = blk * BS + threadIdx.x; ip < n; ip += RED_GRID * BS)
+    for (int ip = blk * BS + threadIdx.x; ip < n; ip += gridDim.x * BS)
         acc[0] += (A.dx[ip % A.nx] * A.dy[ip / A.nx]) * r[ip];
     block_sum<1>(acc);
     if (threadIdx.x == 0) part[blk] = acc[0];
@@ -395,13 +386,21 @@ PoissonStencil::PoissonStencil(const GridDev &g, double dt, bool centre_pin, hip
 
 void PoissonStencil::spmv_dot(const double *x, double *y, const double *a, bool want_yy, double *part,
                               hipStream_t s) const {
-    hipLaunchKernelGGL(k_p5_spmv_dot, dim3(RED_GRID), dim3(BS), 0, s, dev(), x, y, a, (int)want_yy, part);
+    hipLaunchKernelGGL(k_p5_spmv_dot<false>, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), x, nullptr, nullptr, y, a,
+                       (int)want_yy, FinArgs{}, part);
+    CUIBM_LAUNCH_CHECK();
+}
+
+void PoissonStencil::spmv_dot_jacobi(const double *dinv, const double *p, double *Mp, double *y, const double *a,
+                                     bool want_yy, const FinArgs &f, double *part, hipStream_t s) const {
+    hipLaunchKernelGGL(k_p5_spmv_dot<true>, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), p, dinv, Mp, y, a,
+                       (int)want_yy, f, part);
     CUIBM_LAUNCH_CHECK();
 }
 
 void PoissonStencil::init(const double *x, const double *b, double *r, double *p, double *rs, double *part,
                           hipStream_t s) const {
-    hipLaunchKernelGGL(k_p5_init, dim3(RED_GRID), dim3(BS), 0, s, dev(), x, b, r, p, rs, part);
+    hipLaunchKernelGGL(k_p5_init, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), x, b, r, p, rs, part);
     CUIBM_LAUNCH_CHECK();
 }
 
@@ -456,34 +455,43 @@ __global__ void k_v5_coef(int nx, int ny, const double *__restrict__ dx, const d
     }
 }
 
-// (LHS1 x)_i for the packed index i, in the CSR column order S, W, C, E, N
-__device__ __forceinline__ double v5_row(const V5Dev &A, int i, const double *__restrict__ x) {
+// (LHS1 x)_i for the packed index i, in the CSR column order S, W, C, E, N; x(j) gives x_j
+template <class F>
+__device__ __forceinline__ double v5_row(const V5Dev &A, int i, F x) {
     const V5Block &B = i < A.v.off0 ? A.u : A.v;
     const int k = i - B.off0, I = k % B.ni, J = k / B.ni;
     const double d = (((1.0 + B.dE[I]) + B.dW[I]) + B.dN[J]) + B.dS[J];
     double s = 0;
-    if (J != 0) s += (-B.oS[J]) * x[i - B.ni];
-    if (I != 0) s += (-B.oW[I]) * x[i - 1];
-    s += d * x[i];
-    if (I != B.ni - 1) s += (-B.oE[I]) * x[i + 1];
-    if (J != B.nj - 1) s += (-B.oN[J]) * x[i + B.ni];
+    if (J != 0) s += (-B.oS[J]) * x(i - B.ni);
+    if (I != 0) s += (-B.oW[I]) * x(i - 1);
+    s += d * x(i);
+    if (I != B.ni - 1) s += (-B.oE[I]) * x(i + 1);
+    if (J != B.nj - 1) s += (-B.oN[J]) * x(i + B.ni);
     return s;
 }
 
-// y = A x with block partials of (y . a) and (y . y): the loop, grid and reduction of
-// the CSR k_spmv_dot, so the partials are the CSR path's
+// y = A x with block partials of (y . a) and (y . y); JAC as in k_p5_spmv_dot
+template <bool JAC>
 __global__ void __launch_bounds__(BS) k_v5_spmv_dot(V5Dev A, int n, const double *__restrict__ x,
+                                                    const double *__restrict__ dinv, double *__restrict__ Mp,
                                                     double *__restrict__ y, const double *__restrict__ a, int want_yy,
-                                                    double *__restrict__ part) {
+                                                    FinArgs f, double *__restrict__ part) {
     const double stopv = A.stop ? *A.stop : 0.0;  // the Krylov solve's stop code, tested after the loads
+    if (JAC && f.part) {
+        double tot[2] = {0, 0};
+        finish_sums<1>(f, tot);
+        if (stopv != 0.0) return;  // uniform, as every return before the last barrier
+        if (fin_ss(tot, f.sc, blockIdx.x == 0 && threadIdx.x == 0) != 0.0) return;
+    }
     double acc[2] = {0, 0};
     bool tested = false;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double yi = v5_row(A, i, x);
+        const double yi = v5_row(A, i, [&](int j) { return JAC ? dinv[j] * x[j] : x[j]; });
         if (!tested) {
             if (stopv != 0.0) return;  // every thread returns here or below: no barrier is reached
             tested = true;
         }
+        if (JAC) Mp[i] = dinv[i] * x[i];
         if (y) y[i] = yi;
         acc[0] += yi * a[i];
         acc[1] += yi * yi;
@@ -504,7 +512,7 @@ __global__ void __launch_bounds__(BS) k_v5_init(V5Dev A, int n, const double *__
     double acc[2] = {0, 0};
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const double bi = b[i];
-        const double ri = bi - v5_row(A, i, x);
+        const double ri = bi - v5_row(A, i, [&](int j) { return x[j]; });
         r[i] = ri;
         p[i] = ri;
         rs[i] = ri;
@@ -539,13 +547,21 @@ V5Dev VelocityStencil::dev() const {
 
 void VelocityStencil::spmv_dot(const double *x, double *y, const double *a, bool want_yy, double *part,
                                hipStream_t s) const {
-    hipLaunchKernelGGL(k_v5_spmv_dot, dim3(RED_GRID), dim3(BS), 0, s, dev(), n(), x, y, a, (int)want_yy, part);
+    hipLaunchKernelGGL(k_v5_spmv_dot<false>, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), n(), x, nullptr, nullptr, y,
+                       a, (int)want_yy, FinArgs{}, part);
+    CUIBM_LAUNCH_CHECK();
+}
+
+void VelocityStencil::spmv_dot_jacobi(const double *dinv, const double *p, double *Mp, double *y, const double *a,
+                                      bool want_yy, const FinArgs &f, double *part, hipStream_t s) const {
+    hipLaunchKernelGGL(k_v5_spmv_dot<true>, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), n(), p, dinv, Mp, y, a,
+                       (int)want_yy, f, part);
     CUIBM_LAUNCH_CHECK();
 }
 
 void VelocityStencil::init(const double *x, const double *b, double *r, double *p, double *rs, double *part,
                            hipStream_t s) const {
-    hipLaunchKernelGGL(k_v5_init, dim3(RED_GRID), dim3(BS), 0, s, dev(), n(), x, b, r, p, rs, part);
+    hipLaunchKernelGGL(k_v5_init, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), n(), x, b, r, p, rs, part);
     CUIBM_LAUNCH_CHECK();
 }
 
@@ -577,7 +593,7 @@ void launch_p5_sweep2(const P5Dev &A, double omega, const double *x, const doubl
 
 void launch_p5_wdot(const P5Dev &A, const double *r, double *part, hipStream_t s) {
     if (!A.dx || !A.dy) throw Error("the constant mode needs the cell widths of the stencil operator", ERR_ARGUMENT);
-    hipLaunchKernelGGL(k_p5_wdot, dim3(RED_GRID), dim3(BS), 0, s, A, r, part);
+    hipLaunchKernelGGL(k_p5_wdot, dim3(red_blocks((long)A.nx * A.ny)), dim3(BS), 0, s, A, r, part);
     CUIBM_LAUNCH_CHECK();
 }
 
@@ -593,7 +609,7 @@ int p5_tiles(int nx, int ny) { return ((nx + TX - 1) / TX) * ((ny + TY - 1) / TY
 
 template <int OP>
 __device__ __forceinline__ double b_row(const BCase &C, int i, const double *__restrict__ xc) {
-    if (OP == BOP_VEL) return v5_row(C.v5, i, xc);
+    if (OP == BOP_VEL) return v5_row(C.v5, i, [&](int j) { return xc[j]; });
     const P5Dev &A = C.p5;
     const int I = i % A.nx, J = i / A.nx;
     return p5_row(A, I, J, p5_diag(A, I, J, i), [&](int o) { return xc[i + o]; }, A.nx);

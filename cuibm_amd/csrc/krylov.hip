@@ -4,9 +4,9 @@
 // Right-preconditioned BiCGSTAB (van der Vorst 1992) with the monitor rule
 // ||r||_2 <= rtol ||b||_2 checked on r before every iteration and on s half-way
 // through it; the iteration count counts full iterations. The recurrence scalars
-// (rho, alpha, omega, beta) never leave the GPU: reductions finish in a one-block
-// kernel that updates them in place, and the host reads back the scalar block twice
-// per iteration for the stopping test.
+// (rho, alpha, omega, beta) never leave the GPU: reductions finish in the kernel that needs
+// the result, or in a one-block kernel, and update them in place; the stopping tests run
+// there too, and the host reads the scalar block back once per batch of queued iterations.
 //
 // Breakdown (alpha or ||s|| not finite, omega = 0, rho = 0, beta not finite) restarts
 // the recurrence from the true residual b - A x of the current iterate, keeping the
@@ -70,52 +70,80 @@ Bicgstab::~Bicgstab() {
 SolveStat Bicgstab::solve(const LinOp &A, double *x, const double *b, Preconditioner &M, double rtol,
                           int maxit, hipStream_t s) {
     if (A.n() != n_) throw Error("BiCGSTAB workspace size mismatch", ERR_ARGUMENT);
-    const int n = n_;
-    double *sc = sc_, *part = part_;
-    const double *stop = sc + SC_STOP;
-    A.set_stop(stop);
-    M.set_stop(stop);
+    const int n = n_, np = red_blocks(n);
+    // small systems: every reduction is finished by the kernel that uses it (FinArgs), from the
+    // half of the partials that this kernel does not write
+    const bool fused = np <= FUSE_PARTS;
+    double *sc = sc_, *part0 = part_, *part1 = fused ? part_ + FUSE_PARTS : part_;
+    const double *diag = M.diagonal();
+    int par = 0;  // parity of the iteration since the last (re)start
+    auto args = [&](const double *part) { return FinArgs{fused ? part : nullptr, np, sc, par, maxit}; };
+    auto finish = [&](const double *part, int op) { launch_bicg_finish(part, np, op, args(nullptr), s, rtol); };
     SolveStat st;
     auto fetch = [&]() {  // the scalar block: one small copy, one sync
-        CUIBM_HIP(hipMemcpyAsync(host_sc_, sc, SC_D0 * sizeof(double), hipMemcpyDeviceToHost, s));
+        CUIBM_HIP(hipMemcpyAsync(host_sc_, sc, SC_COUNT * sizeof(double), hipMemcpyDeviceToHost, s));
         CUIBM_HIP(hipStreamSynchronize(s));
     };
-    auto start = [&]() {  // r = b - A x, rs = p = r; clears the stop code
-        A.init(x, b, r_, p_, rs_, part, s);
-        launch_bicg_finish(part, FIN_INIT, sc, s);
-        fetch();
+    auto start = [&](int op) {  // r = b - A x, rs = p = r; clears the stop codes
+        par = 0;
+        A.init(x, b, r_, p_, rs_, part0, s);
+        finish(part0, op);
     };
-    launch_fill(sc + SC_ITS, 0.0, 1, s);
-    start();
-    const double tol = rtol * std::sqrt(host_sc_[SC_BB]);
-    double rn = std::sqrt(host_sc_[SC_RR]);
-    const double rn0 = rn;
-    int it = 0, restarts = 0;
-    st.tolerance = tol;
-    // the first half of iteration k (through the test on ||s||), then the second half.
-    // A preconditioner that forms weighted sums of its input gets them from the kernels
+    // the first half of iteration k (through s, and the test on ||s|| if `test`), then the second
+    // half. A preconditioner that forms weighted sums of its input gets them from the kernels
     // that produce s and p (for the p of a (re)start, it forms them itself).
     const InputWeights iw = M.input_weights();
     const InputWeights *wp = iw.part ? &iw : nullptr;
     bool p_weighted = false;
-    auto half1 = [&]() {
-        if (wp && p_weighted) M.apply_weighted(p_, Mp_, s);
-        else M.apply(p_, Mp_, s);
-        A.spmv_dot(Mp_, AMp_, rs_, false, part, s);
-        launch_bicg_finish(part, FIN_ALPHA, sc, s);
-        launch_bicg_s(n, r_, AMp_, s_, sc, part, s, wp);
-        launch_bicg_finish(part, FIN_SS, sc, s, tol, maxit);
+    auto half1 = [&](bool test) {
+        const double *stop = sc + sc_stop(par);
+        A.set_stop(stop);
+        M.set_stop(stop);
+        if (diag) {
+            A.spmv_dot_jacobi(diag, p_, Mp_, AMp_, rs_, false, FinArgs{}, part0, s);
+        } else {
+            if (wp && p_weighted) M.apply_weighted(p_, Mp_, s);
+            else M.apply(p_, Mp_, s);
+            A.spmv_dot(Mp_, AMp_, rs_, false, part0, s);
+        }
+        if (!fused) finish(part0, FIN_ALPHA);
+        launch_bicg_s(n, r_, AMp_, s_, args(part0), part1, s, wp);
+        if (test) finish(part1, FIN_SS);
     };
-    auto half2 = [&]() {
-        if (wp) M.apply_weighted(s_, Ms_, s);
-        else M.apply(s_, Ms_, s);
-        A.spmv_dot(Ms_, AMs_, s_, true, part, s);
-        launch_bicg_finish(part, FIN_OMEGA, sc, s);
-        launch_bicg_xr(n, x, Mp_, Ms_, r_, s_, AMs_, rs_, sc, part, s);
-        launch_bicg_finish(part, FIN_BETA, sc, s, tol, maxit);
-        launch_bicg_p(n, p_, r_, AMp_, sc, s, wp);
+    auto half2 = [&](bool tested) {
+        const double *stop = sc + (tested ? (int)SC_STOPS : sc_stop(par));  // FIN_SS hands the other on
+        A.set_stop(stop);
+        M.set_stop(stop);
+        if (diag) {
+            A.spmv_dot_jacobi(diag, s_, Ms_, AMs_, s_, true, tested ? FinArgs{} : args(part1), part0, s);
+        } else {
+            if (wp) M.apply_weighted(s_, Ms_, s);
+            else M.apply(s_, Ms_, s);
+            A.spmv_dot(Ms_, AMs_, s_, true, part0, s);
+        }
+        if (!fused) finish(part0, FIN_OMEGA);
+        launch_bicg_xr(n, x, Mp_, Ms_, r_, s_, AMs_, rs_, args(part0), part1, s);
+        if (!fused) finish(part1, FIN_BETA);
+        launch_bicg_p(n, p_, r_, AMp_, args(part1), s, wp);
         p_weighted = wp != nullptr;
+        par ^= 1;
     };
+    const bool test_early = !(diag && fused);  // ||s|| is tested before the second product (else in it)
+    start(FIN_INIT);
+    double tol = 0, rn = 0, rn0 = 0, rn_ref = 0;
+    // with an earlier solve to go by, iterations are queued before the first read-back
+    bool known = false;
+    auto first_known = [&]() {
+        tol = host_sc_[SC_TOL];
+        rn0 = rn_ref = std::sqrt(host_sc_[SC_D0]);
+        known = true;
+    };
+    if (exact_ || last_its_ < 0 || maxit <= 0) {
+        fetch();
+        first_known();
+        rn = rn0;
+    }
+    int it = 0, restarts = 0;
     // The recurrence residual r can drift from b - A x through rounding when a solve runs
     // many iterations with large updates (seen with the FP32 V-cycle at tolerances near
     // 1e-12: after thousands of iterations r claimed 5e-11 of ||b|| while b - A x was
@@ -123,38 +151,55 @@ SolveStat Bicgstab::solve(const LinOp &A, double *x, const double *b, Preconditi
     // therefore forms b - A x once; more than kDriftFactor times the tolerance restarts
     // the iteration from it (counted as a restart), at most kMaxChecks times.
     int checks = 0;
-    const double reliable = M.restart_reduction();
-    double rn_ref = rn;  // the true residual at the last (re)start
+    const double reliable = M.restart_reduction();  // rn_ref: the true residual at the last (re)start
+    auto restart = [&]() {
+        start(FIN_RESTART);
+        fetch();
+        p_weighted = false;
+        return std::sqrt(host_sc_[SC_RR]);
+    };
     for (;;) {
-        while (!(rn <= tol) && it < maxit) {
+        while (!known || (!(rn <= tol) && it < maxit)) {
             // iterations to queue before the next read-back: a fraction of the estimate from
             // the residual reduction so far (or of the last solve), so that few launches
             // fall past the end; one in exact mode
             int batch = 1;
+            // a solve that will likely leave at its first half step is read back there
+            const bool stepwise = exact_ || (!known && last_its_ == 0);
             if (!exact_) {
-                double rate = rate_;
-                if (it > 0 && rn < rn0) rate = std::pow(rn / rn0, 1.0 / it);
-                if (rate > 0 && rate < 1) {
-                    const double left = std::log(tol / rn) / std::log(rate);
-                    batch = (int)std::max(1.0, std::min(16.0, std::floor(0.7 * left)));
+                double left = 0;
+                if (!known) {
+                    left = last_its_;
+                } else {
+                    double rate = rate_;
+                    if (it > 0 && rn < rn0) rate = std::pow(rn / rn0, 1.0 / it);
+                    if (rate > 0 && rate < 1) left = std::log(tol / rn) / std::log(rate);
                 }
+                batch = (int)std::max(1.0, std::min(16.0, std::floor(0.7 * left)));
                 batch = std::min(batch, maxit - it);
             }
+            int code = 0;
             for (int j = 0; j < batch; j++) {
-                half1();
-                if (exact_) {  // no launch past a half-step exit or breakdown
+                half1(test_early || stepwise);
+                if (stepwise) {  // no launch past a half-step exit or breakdown
                     fetch();
-                    if (host_sc_[SC_STOP] == STOP_HALF_PENDING) {  // the half-step update alone
-                        launch_bicg_xr(n, x, Mp_, Ms_, r_, s_, AMs_, rs_, sc, part, s);
-                        launch_bicg_finish(part, FIN_BETA, sc, s, tol, maxit);
+                    const int h = (int)host_sc_[SC_STOPS], c = (int)host_sc_[sc_stop(par)];
+                    if (c == 0 && h == STOP_HALF_PENDING) {  // the half-step update alone
+                        launch_bicg_xr(n, x, Mp_, Ms_, r_, s_, AMs_, rs_, FinArgs{nullptr, np, sc, par, maxit}, part1, s);
+                        code = STOP_HALF;
+                    } else if (c != 0 || h != 0) {
+                        code = c != 0 ? c : h;
                     }
-                    if (host_sc_[SC_STOP] != 0.0) break;
+                    if (code != 0) break;
                 }
-                half2();
+                half2(test_early || stepwise);
             }
-            fetch();
+            if (code == 0) {
+                fetch();
+                code = (int)host_sc_[sc_stop(par)];
+            }
+            if (!known) first_known();
             it = (int)host_sc_[SC_ITS];
-            const int code = (int)host_sc_[SC_STOP];
             if (code == STOP_HALF) {
                 rn = std::sqrt(host_sc_[SC_SS]);
                 break;
@@ -162,31 +207,27 @@ SolveStat Bicgstab::solve(const LinOp &A, double *x, const double *b, Preconditi
             rn = std::sqrt(host_sc_[SC_RR]);
             if (code == STOP_BREAK_HALF || code == STOP_BREAK_FULL) {
                 if (++restarts > kMaxRestarts) break;
-                start();  // x is untouched by a half-step breakdown
-                p_weighted = false;
-                rn = rn_ref = std::sqrt(host_sc_[SC_RR]);
+                rn = rn_ref = restart();  // x is untouched by a half-step breakdown
             } else if (reliable > 0 && code == 0 && rn < reliable * rn_ref) {
                 if (++restarts > kMaxRestarts) break;
-                start();  // reliable update: the true residual, new search directions
-                p_weighted = false;
-                rn = rn_ref = std::sqrt(host_sc_[SC_RR]);
+                rn = rn_ref = restart();  // reliable update: the true residual, new search directions
             }
         }
         if (!(rn <= tol) || (it < kVerifyIts && restarts == 0) || checks >= kMaxChecks) break;
         checks++;
-        start();
-        p_weighted = false;
-        const double tr = std::sqrt(host_sc_[SC_RR]);
+        const double tr = restart();
         if (tr <= kDriftFactor * tol) break;
         rn = rn_ref = tr;
         if (++restarts > kMaxRestarts) break;
     }
     if (it > 0 && rn > 0 && rn0 > 0 && rn < rn0) rate_ = std::pow(rn / rn0, 1.0 / it);
+    last_its_ = it;
     A.set_stop(nullptr);
     M.set_stop(nullptr);
     st.restarts = restarts;
     st.iterations = it;
     st.residual = rn;
+    st.tolerance = tol;
     st.converged = rn <= tol;
     return st;
 }

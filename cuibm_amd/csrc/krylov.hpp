@@ -9,22 +9,48 @@
 
 namespace cuibm {
 
-constexpr int RED_GRID = 2048;  // blocks of every reducing kernel
+constexpr int RED_GRID = 2048;  // most blocks of a reducing kernel, and partial sums of one group
+// blocks of the reducing kernels of n unknowns: one block per BS unknowns (a multiple of 8, see
+// xcd_block) up to RED_GRID, which stride over the vector. The partials do not depend on it:
+// blocks without an unknown would add zeros.
+inline int red_blocks(long n) { return (int)std::min<long>(RED_GRID, (n / BS + 8) / 8 * 8); }
 
 // slots of the device scalar block. SC_STOP is the device-side end of the iteration:
 // 0 running, STOP_* below otherwise; every kernel of the iteration returns at once when
 // it is set, so the host may queue several iterations before reading the block back.
 enum { SC_BB = 0, SC_RHO, SC_ALPHA, SC_OMEGA, SC_BETA, SC_SS, SC_RR, SC_STOP, SC_ITS, SC_HALFK, SC_D0, SC_D1,
-       SC_TOL, SC_COUNT = 16 };  // SC_TOL: the absolute tolerance of a batched solve
+       SC_TOL, SC_RHO2, SC_STOP2, SC_STOPS, SC_COUNT = 16 };
+// SC_TOL: the absolute tolerance. A single solve keeps rho and the stop code in one slot per
+// parity of the iteration (iteration k reads k & 1 and writes the other) and the half step's stop
+// code in SC_STOPS; SC_D0 holds r.r of the first residual. Batched solves use the first slots.
+inline __host__ __device__ int sc_rho(int par) { return par ? SC_RHO2 : SC_RHO; }
+inline __host__ __device__ int sc_stop(int par) { return par ? SC_STOP2 : SC_STOP; }
 // STOP_HALF_PENDING: the half step converged in this iteration and the x update of its
 // second half is still due (the iteration's FIN_BETA finish turns it into STOP_HALF), so
 // the launches of an iteration do not depend on its index
 enum { STOP_CONVERGED = 1, STOP_HALF = 2, STOP_BREAK_HALF = 3, STOP_BREAK_FULL = 4, STOP_MAXIT = 5,
        STOP_HALF_PENDING = 6 };
 // finish-kernel operations
-// FIN_RESTART (batched solves): a restart of the cases marked in a mask, from the true
-// residual; the iteration count, the tolerance and the half-step record are kept
-enum { FIN_INIT = 0, FIN_ALPHA, FIN_SS, FIN_OMEGA, FIN_BETA, FIN_DOT2, FIN_RESTART };
+// FIN_RESTART: a restart (in a batch, of the cases marked in a mask) from the true residual;
+// the iteration count, the tolerance and the half-step record are kept
+enum { FIN_INIT = 0, FIN_ALPHA, FIN_SS, FIN_OMEGA, FIN_BETA, FIN_RESTART };
+
+// The finish of a reduction inside the kernel that uses its result: with `part` the kernel adds
+// the np partials there itself (every block, in k_bicg_finish's order) and one thread stores
+// the scalars, without it a finish launch has. A launch costs 3.5-4 us whatever it does, the
+// sums about 1 us of the consumer for a few hundred partials; beyond FUSE_PARTS every block reading
+// them all costs more (462^2, 840 partials: the x and r update 11.7 us against 5 and a finish of
+// 3, an embedded step 7.8 ms unfused against 8.6). The kernel's own partials go to another half
+// of the buffer. Steps with finishes, Jacobi products and first read-backs fused, before and
+// after: 32^2 cavity 0.29 -> 0.18 ms, 128^2 1.08 -> 0.77, 336^2 cylinder (FP64) 3.1 -> 2.7.
+constexpr int FUSE_PARTS = 512;
+struct FinArgs {
+    const double *part = nullptr;
+    int np = 0;
+    double *sc = nullptr;  // scalar block
+    int par = 0;           // parity of the iteration
+    int maxit = 0;
+};
 
 // ---- k_blas.hip
 void launch_fill(double *x, double v, long n, hipStream_t s);
@@ -37,6 +63,9 @@ template <class V, class X>
 void launch_spmv(const DCsr<V> &A, const X *x, X *y, hipStream_t s);
 void launch_spmv_dot(const DCsr<double> &A, const double *x, double *y, const double *a, bool want_yy, double *part,
                      hipStream_t s, const double *stop = nullptr);
+void launch_spmv_dot_jacobi(const DCsr<double> &A, const double *dinv, const double *p, double *Mp, double *y,
+                            const double *a, bool want_yy, const FinArgs &f, double *part, hipStream_t s,
+                            const double *stop);
 void launch_bicg_init(const DCsr<double> &A, const double *x, const double *b, double *r, double *p, double *rs,
                       double *part, hipStream_t s);
 // weights w_i = wx[i % nx] * wy[i / nx] of a preconditioner's input (cell areas), whose
@@ -46,20 +75,20 @@ struct InputWeights {
     int nx = 0;
     double *part = nullptr;
 };
-// s = r - alpha AMp with partials of (s.s); with w, also the weighted partials of s
-void launch_bicg_s(int n, const double *r, const double *AMp, double *s_, const double *sc, double *part, hipStream_t s,
+// s = r - alpha AMp (after FIN_ALPHA) with partials of (s.s); with w, also the weighted partials
+void launch_bicg_s(int n, const double *r, const double *AMp, double *s_, const FinArgs &f, double *part, hipStream_t s,
                    const InputWeights *w = nullptr);
-// x += alpha Mp + omega Ms, r = s - omega AMs with partials; after a half-step exit of
-// the same iteration (STOP_HALF_PENDING), x += alpha Mp only
+// x += alpha Mp + omega Ms, r = s - omega AMs (after FIN_OMEGA) with partials; after a half-step
+// exit of the same iteration (STOP_HALF_PENDING), x += alpha Mp only
 void launch_bicg_xr(int n, double *x, const double *Mp, const double *Ms, double *r, const double *s_,
-                    const double *AMs, const double *rs, const double *sc, double *part, hipStream_t s);
-// p = r + beta (p - omega AMp); with w, also the weighted partials of p
-void launch_bicg_p(int n, double *p, const double *r, const double *AMp, const double *sc, hipStream_t s,
+                    const double *AMs, const double *rs, const FinArgs &f, double *part, hipStream_t s);
+// p = r + beta (p - omega AMp) (after FIN_BETA); with w, also the weighted partials of p
+void launch_bicg_p(int n, double *p, const double *r, const double *AMp, const FinArgs &f, hipStream_t s,
                    const InputWeights *w = nullptr);
-// sums the partials and updates the scalars; FIN_SS and FIN_BETA also apply the stopping
-// tests of the monitor (tol) and the iteration limit (maxit) and set SC_STOP
-void launch_bicg_finish(const double *part, int op, double *sc, hipStream_t s, double tol = 0, int maxit = 0);
-void launch_dot2(long n, const double *x, const double *y, double *part, hipStream_t s);
+// one block: sums the np partials of each group and updates the scalars of iteration parity
+// f.par; FIN_INIT also forms the tolerance rtol ||b||, FIN_SS and FIN_BETA apply the stopping
+// tests of the monitor and the iteration limit
+void launch_bicg_finish(const double *part, int np, int op, const FinArgs &f, hipStream_t s, double rtol = 0);
 void launch_jacobi_apply(int n, const double *dinv, const double *r, double *z, hipStream_t s,
                          const double *stop = nullptr);
 void launch_diag_inv(const DCsr<double> &A, double *dinv, hipStream_t s);
@@ -72,6 +101,11 @@ class LinOp {
     // y = A x (y may be null) with partials of (y . a) and, if want_yy, (y . y)
     virtual void spmv_dot(const double *x, double *y, const double *a, bool want_yy, double *part,
                           hipStream_t s) const = 0;
+    // Mp = D^-1 p and y = A Mp in one launch, with the same partials: the Jacobi preconditioner
+    // as part of the product (each point's D^-1 p formed at its neighbours, the same bits). With
+    // f.part, after FIN_SS.
+    virtual void spmv_dot_jacobi(const double *dinv, const double *p, double *Mp, double *y, const double *a,
+                                 bool want_yy, const FinArgs &f, double *part, hipStream_t s) const = 0;
     // r = b - A x, p = rs = r, partials of (r . r) and (b . b)
     virtual void init(const double *x, const double *b, double *r, double *p, double *rs, double *part,
                       hipStream_t s) const = 0;
@@ -91,6 +125,10 @@ class CsrOp : public LinOp {
     void spmv_dot(const double *x, double *y, const double *a, bool want_yy, double *part,
                   hipStream_t s) const override {
         launch_spmv_dot(A_, x, y, a, want_yy, part, s, stop_);
+    }
+    void spmv_dot_jacobi(const double *dinv, const double *p, double *Mp, double *y, const double *a, bool want_yy,
+                         const FinArgs &f, double *part, hipStream_t s) const override {
+        launch_spmv_dot_jacobi(A_, dinv, p, Mp, y, a, want_yy, f, part, s, stop_);
     }
     void init(const double *x, const double *b, double *r, double *p, double *rs, double *part,
               hipStream_t s) const override {
@@ -116,6 +154,8 @@ class Preconditioner {
     // the true residual b - A x whenever its residual has fallen by this factor since the
     // last (re)start (reliable updates); 0: never
     virtual double restart_reduction() const { return 0.0; }
+    // the inverse diagonal of a Jacobi preconditioner: the products then apply it themselves
+    virtual const double *diagonal() const { return nullptr; }
     virtual std::string name() const = 0;
     // bytes moved by one apply, counted as distinct arrays touched per kernel
     virtual double bytes_per_apply() const = 0;
@@ -146,6 +186,7 @@ class JacobiPrecond : public Preconditioner {
     void apply(const double *r, double *z, hipStream_t s) override;
     // D^-1 of a new matrix of the same size, in place
     void refresh(const DCsr<double> &A, hipStream_t s);
+    const double *diagonal() const override { return dinv_; }
     std::string name() const override { return "DIAGONAL"; }
     double bytes_per_apply() const override { return 24.0 * n_; }
 
@@ -375,6 +416,7 @@ class Bicgstab {
     int n_;
     bool exact_ = false;
     double rate_ = 0;  // mean residual reduction per iteration of the last solve
+    int last_its_ = -1;  // its full iterations; -1: none yet
     DArray<double> own_;
     double *r_ = nullptr, *rs_ = nullptr, *p_ = nullptr, *Mp_ = nullptr, *AMp_ = nullptr, *s_ = nullptr,
            *Ms_ = nullptr, *AMs_ = nullptr, *part_ = nullptr, *sc_ = nullptr;

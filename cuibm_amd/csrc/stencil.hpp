@@ -30,6 +30,8 @@ class PoissonStencil : public LinOp {
     int n() const override { return nx_ * ny_; }
     void spmv_dot(const double *x, double *y, const double *a, bool want_yy, double *part,
                   hipStream_t s) const override;
+    void spmv_dot_jacobi(const double *dinv, const double *p, double *Mp, double *y, const double *a, bool want_yy,
+                         const FinArgs &f, double *part, hipStream_t s) const override;
     void init(const double *x, const double *b, double *r, double *p, double *rs, double *part,
               hipStream_t s) const override;
     double spmv_bytes() const override { return 16.0 * n() + 32.0 * (nx_ + ny_); }
@@ -72,6 +74,8 @@ class VelocityStencil : public LinOp {
     int n() const override { return nu_ + nv_; }
     void spmv_dot(const double *x, double *y, const double *a, bool want_yy, double *part,
                   hipStream_t s) const override;
+    void spmv_dot_jacobi(const double *dinv, const double *p, double *Mp, double *y, const double *a, bool want_yy,
+                         const FinArgs &f, double *part, hipStream_t s) const override;
     void init(const double *x, const double *b, double *r, double *p, double *rs, double *part,
               hipStream_t s) const override;
     double spmv_bytes() const override { return 16.0 * n() + 64.0 * (nx_ + ny_); }
@@ -89,7 +93,7 @@ class VelocityStencil : public LinOp {
 void launch_p5_pre(const P5Dev &A, double omega, const double *b, double *x2, double *r, hipStream_t s,
                    KernelProbe *probe = nullptr);
 void launch_p5_sweep2(const P5Dev &A, double omega, const double *x, const double *b, double *xo, hipStream_t s);
-// partial sums of w_i r_i (w = cell areas) over RED_GRID blocks, for the constant mode of a
+// red_blocks(n) partial sums of w_i r_i (w = cell areas), for the constant mode of a
 // multigrid input (mg.hpp); returns at once while the Krylov solve's stop code is set
 void launch_p5_wdot(const P5Dev &A, const double *r, double *part, hipStream_t s);
 // one sweep xn = x + omega D^-1 (b - A x) (timing of the finest-level smoother)
