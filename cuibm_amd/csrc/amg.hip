@@ -1280,7 +1280,7 @@ struct BatchAmg::Impl {
 };
 
 BatchAmg::BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long> &offP, const BCase *tab_dev,
-                   const std::vector<BCase> &tab_host, const BMapDev &pmap, const int *pfirst, hipStream_t s)
+                   const std::vector<BCase> &tab_host, const std::vector<int> &nblk, hipStream_t s)
     : im_(new Impl) {
     if (amg.empty()) throw Error("batched V-cycle without cases", ERR_ARGUMENT);
     const int prec = amg[0]->precision();
@@ -1293,7 +1293,7 @@ BatchAmg::BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long>
     if (prec != 64 && prec != 32) throw Error("batched V-cycle: AMG precision 64 or 32", ERR_UNSUPPORTED);
     if (!mg.empty() && mg.size() != amg.size()) throw Error("batched V-cycle: cases of different hierarchies", ERR_ARGUMENT);
     if (!mg.empty()) {
-        im_->mg.reset(new BatchMg(mg, offP, tab_dev, tab_host, pmap, pfirst, s));
+        im_->mg.reset(new BatchMg(mg, offP, tab_host, nblk, s));
         return;
     }
     const int n = (int)amg.size();
@@ -1318,6 +1318,8 @@ void BatchAmg::apply(const double *r, double *z, hipStream_t s) {
     if (im_->mg) im_->mg->apply(r, z, s);
     else im_->d64.apply(r, z, s);
 }
+
+double *BatchAmg::weights_part() const { return im_->mg ? im_->mg->weights_part() : nullptr; }
 
 int BatchAmg::levels() const { return im_->mg ? im_->mg->levels() : (int)im_->d64.lv.size(); }
 

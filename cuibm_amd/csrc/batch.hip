@@ -122,10 +122,14 @@ struct LockstepBatch::Impl {
     DArray<double> fpart, fout;
     double tol1 = 0, tol2 = 0;
     int maxit1 = 0, maxit2 = 0;
-    // eight BiCGSTAB iterations of each operator as one captured graph
-    static constexpr int GRAPH_ITS = 8;
+    // the two halves of a BiCGSTAB iteration of each operator as captured graphs
     bool graphs = true;
-    hipGraphExec_t block[2] = {nullptr, nullptr};
+    hipGraphExec_t half[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+    // iterations queued before a read-back: at first as many as the slowest case of the last solve
+    // took, then a quarter of that (blocks of eight, whatever the solves took, left 7.5 iterations of
+    // launches past the end of every directly preconditioned Poisson solve)
+    static constexpr int MOST_ITS = 8;
+    int last_its[2] = {-1, -1};
     // reliable updates of the Poisson solve (the cases' restart_reduction()): a case whose
     // residual has fallen by this factor since its last (re)start restarts from b - A x
     double reliable2 = 0.0;  // the factor squared (compared with r.r)
@@ -133,8 +137,9 @@ struct LockstepBatch::Impl {
     std::vector<int> host_mask;
 
     ~Impl() {
-        for (hipGraphExec_t &g : block)
-            if (g) (void)hipGraphExecDestroy(g);
+        for (auto &op : half)
+            for (hipGraphExec_t &g : op)
+                if (g) (void)hipGraphExecDestroy(g);
     }
 
     void fetch() {
@@ -152,23 +157,62 @@ struct LockstepBatch::Impl {
         const BMapDev md = m.dev();
         launch_b_init(op, tab.p(), md, x, b, w.r.p(), w.p.p(), w.rs.p(), w.part.p(), s);
         launch_b_finish(op, tab.p(), nc, m.first(), md.nblk, w.part.p(), FIN_INIT, rtol, maxit, s);
-        // one iteration: every launch is the same in every iteration (the stop codes and the
-        // half-step state live in the per-case scalar blocks), so a block of them can be
+        double *wpart = op == BOP_POIS ? amg->weights_part() : nullptr;
+        auto weigh_p = [&]() {  // the p of a (re)start has no producer that weighs it
+            if (wpart) launch_b_wdot(tab.p(), md, w.p.p(), wpart, s);
+        };
+        weigh_p();
+        // the halves of an iteration: every launch is the same in every iteration (the stop codes
+        // and the half-step state live in the per-case scalar blocks), so each half can be
         // captured once and replayed
-        auto iteration = [&]() {
-            precond(w.p.p(), w.Mp.p());
-            launch_b_spmv_dot(op, tab.p(), md, w.Mp.p(), w.AMp.p(), w.rs.p(), false, w.part.p(), s);
-            launch_b_finish(op, tab.p(), nc, m.first(), md.nblk, w.part.p(), FIN_ALPHA, rtol, maxit, s);
-            launch_b_bicg_s(op, tab.p(), md, w.r.p(), w.AMp.p(), w.sv.p(), w.part.p(), s);
-            launch_b_finish(op, tab.p(), nc, m.first(), md.nblk, w.part.p(), FIN_SS, rtol, maxit, s);
-            precond(w.sv.p(), w.Ms.p());
-            launch_b_spmv_dot(op, tab.p(), md, w.Ms.p(), w.AMs.p(), w.sv.p(), true, w.part.p(), s);
-            launch_b_finish(op, tab.p(), nc, m.first(), md.nblk, w.part.p(), FIN_OMEGA, rtol, maxit, s);
+        auto fin = [&](int f) { launch_b_finish(op, tab.p(), nc, m.first(), md.nblk, w.part.p(), f, rtol, maxit, s); };
+        auto update_x = [&]() {
             launch_b_bicg_xr(op, tab.p(), md, x, w.Mp.p(), w.Ms.p(), w.r.p(), w.sv.p(), w.AMs.p(), w.rs.p(),
                              w.part.p(), s);
-            launch_b_finish(op, tab.p(), nc, m.first(), md.nblk, w.part.p(), FIN_BETA, rtol, maxit, s);
-            launch_b_bicg_p(op, tab.p(), md, w.p.p(), w.r.p(), w.AMp.p(), s);
+            fin(FIN_BETA);
         };
+        auto launches = [&](int h) {
+            if (h == 0) {
+                precond(w.p.p(), w.Mp.p());
+                launch_b_spmv_dot(op, tab.p(), md, w.Mp.p(), w.AMp.p(), w.rs.p(), false, w.part.p(), s);
+                fin(FIN_ALPHA);
+                launch_b_bicg_s(op, tab.p(), md, w.r.p(), w.AMp.p(), w.sv.p(), w.part.p(), wpart, s);
+                fin(FIN_SS);
+            } else {
+                precond(w.sv.p(), w.Ms.p());
+                launch_b_spmv_dot(op, tab.p(), md, w.Ms.p(), w.AMs.p(), w.sv.p(), true, w.part.p(), s);
+                fin(FIN_OMEGA);
+                update_x();
+                launch_b_bicg_p(op, tab.p(), md, w.p.p(), w.r.p(), w.AMp.p(), wpart, s);
+            }
+        };
+        auto run = [&](int h) {
+            if (!graphs) {
+                launches(h);
+                return;
+            }
+            // a half reads and writes the same arrays every time (x and the operator's
+            // workspace): capture it at its first use
+            hipGraphExec_t &g = half[op == BOP_VEL ? 0 : 1][h];
+            if (!g) {
+                hipGraph_t graph = nullptr;
+                CUIBM_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+                try {
+                    launches(h);
+                } catch (...) {  // leave the stream out of capture mode
+                    hipGraph_t partial = nullptr;
+                    (void)hipStreamEndCapture(s, &partial);
+                    if (partial) (void)hipGraphDestroy(partial);
+                    throw;
+                }
+                CUIBM_HIP(hipStreamEndCapture(s, &graph));
+                const hipError_t e = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
+                (void)hipGraphDestroy(graph);
+                CUIBM_HIP(e);
+            }
+            CUIBM_HIP(hipGraphLaunch(g, s));
+        };
+        int &last = last_its[op == BOP_VEL ? 0 : 1];
         int it = 0;
         const double rel2 = op == BOP_POIS ? reliable2 : 0.0;
         std::vector<double> rr_ref;
@@ -192,6 +236,7 @@ struct LockstepBatch::Impl {
                     launch_b_init(op, tab.p(), md, x, b, w.r.p(), w.p.p(), w.rs.p(), w.part.p(), s, mask.p());
                     launch_b_finish(op, tab.p(), nc, m.first(), md.nblk, w.part.p(), FIN_RESTART, rtol, maxit, s,
                                     mask.p());
+                    weigh_p();
                     fetch();
                     for (int c = 0; c < nc; c++)
                         if (host_mask[c]) rr_ref[c] = scv(c, op)[SC_RR];
@@ -201,31 +246,26 @@ struct LockstepBatch::Impl {
                     if (!running) break;
                 }
             }
-            const int batch = std::min(GRAPH_ITS, maxit - it);
-            if (graphs && batch == GRAPH_ITS) {
-                // the block reads and writes the same arrays every time (x and the
-                // operator's workspace): capture it at its first use
-                hipGraphExec_t &g = block[op == BOP_VEL ? 0 : 1];
-                if (!g) {
-                    hipGraph_t graph = nullptr;
-                    CUIBM_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                    try {
-                        for (int j = 0; j < GRAPH_ITS; j++) iteration();
-                    } catch (...) {  // leave the stream out of capture mode
-                        hipGraph_t partial = nullptr;
-                        (void)hipStreamEndCapture(s, &partial);
-                        if (partial) (void)hipGraphDestroy(partial);
-                        throw;
-                    }
-                    CUIBM_HIP(hipStreamEndCapture(s, &graph));
-                    const hipError_t e = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
-                    (void)hipGraphDestroy(graph);
-                    CUIBM_HIP(e);
+            if (it == 0 && last == 0) {
+                // every case of the last solve left at its first half step: read back there
+                run(0);
+                fetch();
+                bool all = true;
+                for (int c = 0; c < nc; c++) all = all && scv(c, op)[SC_STOP] != 0.0;
+                if (all) {
+                    update_x();  // the pending half-step updates
+                    fetch();
+                    break;
                 }
-                CUIBM_HIP(hipGraphLaunch(g, s));
-                it += GRAPH_ITS;
-            } else {
-                for (int j = 0; j < batch; j++, it++) iteration();
+                run(1);
+                it = 1;
+                continue;
+            }
+            int batch = it == 0 ? (last > 0 ? last : 1) : std::max(1, last / 4);
+            batch = std::min({batch, MOST_ITS, maxit - it});
+            for (int j = 0; j < batch; j++, it++) {
+                run(0);
+                run(1);
             }
         }
         int most = 0;
@@ -239,6 +279,7 @@ struct LockstepBatch::Impl {
                             ERR_NOT_CONVERGED);
             most = std::max(most, (int)v[SC_ITS]);
         }
+        last = most;
         return most;
     }
 };
@@ -418,7 +459,9 @@ LockstepBatch::LockstepBatch(const std::vector<NavierStokesSolver *> &cases, hip
     B.fpart.alloc((size_t)6 * B.nc * BFORCE_BLOCKS);
     B.fout.alloc((size_t)6 * B.nc);
     launch_fill(B.fout.p(), 0.0, 6 * B.nc, s);
-    B.amg.reset(new BatchAmg(A, B.offP, B.tab.p(), B.tab_host, B.mP.dev(), B.mP.first(), s));
+    std::vector<int> nblk(B.nc);
+    for (int c = 0; c < B.nc; c++) nblk[c] = (int)((cP[c] + BS - 1) / BS);
+    B.amg.reset(new BatchAmg(A, B.offP, B.tab.p(), B.tab_host, nblk, s));
     const double f = A[0]->restart_reduction();
     for (auto *a : A)
         if (a->restart_reduction() != f) throw Error("lockstep batch: cases of different -poissonRestart", ERR_ARGUMENT);

@@ -79,13 +79,14 @@ void launch_b_init(int op, const BCase *tab, const BMapDev &m, const double *x, 
 // y = A x with partials of (y.a) [and (y.y)] per block; returns at once for stopped cases
 void launch_b_spmv_dot(int op, const BCase *tab, const BMapDev &m, const double *x, double *y, const double *a,
                        bool want_yy, double *part, hipStream_t s);
+// (with wpart: also the partial sums of the cell areas times the new s, or p, per block)
 void launch_b_bicg_s(int op, const BCase *tab, const BMapDev &m, const double *r, const double *AMp, double *s_,
-                     double *part, hipStream_t s);
+                     double *part, double *wpart, hipStream_t s);
 void launch_b_bicg_xr(int op, const BCase *tab, const BMapDev &m, double *x, const double *Mp, const double *Ms,
                       double *r, const double *s_, const double *AMs, const double *rs, double *part,
                       hipStream_t s);
 void launch_b_bicg_p(int op, const BCase *tab, const BMapDev &m, double *p, const double *r, const double *AMp,
-                     hipStream_t s);
+                     double *wpart, hipStream_t s);
 // per case: sum its blocks' partials and update its scalars (one block per case); FIN_INIT
 // also sets the case's absolute tolerance rtol * ||b|| in SC_TOL
 void launch_b_finish(int op, const BCase *tab, int ncases, const int *first, int nblk, const double *part, int fin,
@@ -99,11 +100,8 @@ void launch_b_force(const BCase *tab, int ncases, const double *u, const double 
                     double *out, hipStream_t s);
 
 // ---- batched finest AMG level (k_stencil.hip) ----
-// the constant mode of each case's input: partial sums of w_i r_i per block (P map) and, per case, c = sum * inv_wa[c]
-// into defl[c]
+// the constant mode of each case's input: partial sums of w_i r_i per block (P map)
 void launch_b_wdot(const BCase *tab, const BMapDev &m, const double *r, double *part, hipStream_t s);
-void launch_b_wdot_finish(const BCase *tab, int ncases, const int *first, const double *part, const double *inv_wa,
-                          double *defl, hipStream_t s);
 // the tile kernels of the finest level per case (tile map: TX x TY tiles per case)
 void launch_b_p5_pre(const BCase *tab, const BMapDev &tiles, double omega, const double *b, double *x2, double *r,
                      hipStream_t s);
@@ -118,10 +116,13 @@ class TensorMg;
 // that has it is one launch, the constant mode is carried per case.
 class BatchMg {
   public:
-    BatchMg(const std::vector<TensorMg *> &mg, const std::vector<long> &offP, const BCase *tab_dev,
-            const std::vector<BCase> &tab_host, const BMapDev &pmap, const int *pfirst, hipStream_t s);
+    // nblk: blocks of each case in the P map, whose partial sums of the weighted input the kernels
+    // that produce the input leave in weights_part()
+    BatchMg(const std::vector<TensorMg *> &mg, const std::vector<long> &offP, const std::vector<BCase> &tab_host,
+            const std::vector<int> &nblk, hipStream_t s);
     ~BatchMg();
     void apply(const double *r, double *z, hipStream_t s);
+    double *weights_part() const;
     int levels() const;
 
   private:
@@ -136,9 +137,10 @@ class BatchMg {
 class BatchAmg {
   public:
     BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long> &offP, const BCase *tab_dev,
-             const std::vector<BCase> &tab_host, const BMapDev &pmap, const int *pfirst, hipStream_t s);
+             const std::vector<BCase> &tab_host, const std::vector<int> &nblk, hipStream_t s);
     ~BatchAmg();
     void apply(const double *r, double *z, hipStream_t s);
+    double *weights_part() const;  // null for stored hierarchies
     int levels() const;
 
   private:
@@ -153,9 +155,9 @@ class NavierStokesSolver;
 // batch's arrays, stepped there, and can be copied back (copy_back).
 class LockstepBatch {
   public:
-    // graphs: run the solves' eight-iteration blocks as captured HIP graphs (one per
-    // operator, captured at its first full block and replayed after) instead of launching
-    // their kernels one by one
+    // graphs: run the halves of the solves' iterations as captured HIP graphs (two per
+    // operator, captured at their first use and replayed after) instead of launching their
+    // kernels one by one
     LockstepBatch(const std::vector<NavierStokesSolver *> &cases, hipStream_t s, bool graphs = true);
     ~LockstepBatch();
     void step();

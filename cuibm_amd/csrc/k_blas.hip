@@ -483,19 +483,25 @@ __device__ __forceinline__ BSeg bseg(int op, const BCase &C) {
 
 __global__ void __launch_bounds__(BS) k_b_bicg_s(int op, const BCase *__restrict__ tab, BMapDev m,
                                                  const double *__restrict__ r, const double *__restrict__ AMp,
-                                                 double *__restrict__ s, double *__restrict__ part) {
-    const BSeg g = bseg(op, tab[m.cs[blockIdx.x]]);
+                                                 double *__restrict__ s, double *__restrict__ part,
+                                                 double *__restrict__ wpart) {
+    const BCase &C = tab[m.cs[blockIdx.x]];
+    const BSeg g = bseg(op, C);
     if (g.sc[SC_STOP] != 0.0) return;
     const double alpha = g.sc[SC_ALPHA];
     const int i = m.loc[blockIdx.x] * BS + threadIdx.x;
-    double acc[1] = {0};
+    double acc[2] = {0, 0};
     if (i < g.n) {
         const double si = r[g.off + i] - alpha * AMp[g.off + i];
         s[g.off + i] = si;
         acc[0] = si * si;
+        if (wpart) acc[1] = (C.g.dx[i % C.g.nx] * C.g.dy[i / C.g.nx]) * si;
     }
-    block_sum<1>(acc);
-    if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
+    block_sum<2>(acc);
+    if (threadIdx.x == 0) {
+        part[blockIdx.x] = acc[0];
+        if (wpart) wpart[blockIdx.x] = acc[1];
+    }
 }
 
 __global__ void __launch_bounds__(BS) k_b_bicg_xr(int op, const BCase *__restrict__ tab, BMapDev m,
@@ -533,15 +539,22 @@ __global__ void __launch_bounds__(BS) k_b_bicg_xr(int op, const BCase *__restric
 
 __global__ void __launch_bounds__(BS) k_b_bicg_p(int op, const BCase *__restrict__ tab, BMapDev m,
                                                  double *__restrict__ p, const double *__restrict__ r,
-                                                 const double *__restrict__ AMp) {
-    const BSeg g = bseg(op, tab[m.cs[blockIdx.x]]);
+                                                 const double *__restrict__ AMp, double *__restrict__ wpart) {
+    const BCase &C = tab[m.cs[blockIdx.x]];
+    const BSeg g = bseg(op, C);
     if (g.sc[SC_STOP] != 0.0) return;
     const double beta = g.sc[SC_BETA], omega = g.sc[SC_OMEGA];
     const int i = m.loc[blockIdx.x] * BS + threadIdx.x;
+    double acc[1] = {0};
     if (i < g.n) {
         const long j = g.off + i;
-        p[j] = r[j] + beta * p[j] - beta * omega * AMp[j];
+        const double v = r[j] + beta * p[j] - beta * omega * AMp[j];
+        p[j] = v;
+        if (wpart) acc[0] = (C.g.dx[i % C.g.nx] * C.g.dy[i / C.g.nx]) * v;
     }
+    if (!wpart) return;  // uniform
+    block_sum<1>(acc);
+    if (threadIdx.x == 0) wpart[blockIdx.x] = acc[0];
 }
 
 // one block per case: the case's block partials in a fixed order, then finish_update
@@ -580,8 +593,8 @@ __global__ void __launch_bounds__(BS) k_b_finish(int op, const BCase *__restrict
 }
 
 void launch_b_bicg_s(int op, const BCase *tab, const BMapDev &m, const double *r, const double *AMp, double *s_,
-                     double *part, hipStream_t s) {
-    hipLaunchKernelGGL(k_b_bicg_s, dim3(m.nblk), dim3(BS), 0, s, op, tab, m, r, AMp, s_, part);
+                     double *part, double *wpart, hipStream_t s) {
+    hipLaunchKernelGGL(k_b_bicg_s, dim3(m.nblk), dim3(BS), 0, s, op, tab, m, r, AMp, s_, part, wpart);
     CUIBM_LAUNCH_CHECK();
 }
 
@@ -593,8 +606,8 @@ void launch_b_bicg_xr(int op, const BCase *tab, const BMapDev &m, double *x, con
 }
 
 void launch_b_bicg_p(int op, const BCase *tab, const BMapDev &m, double *p, const double *r, const double *AMp,
-                     hipStream_t s) {
-    hipLaunchKernelGGL(k_b_bicg_p, dim3(m.nblk), dim3(BS), 0, s, op, tab, m, p, r, AMp);
+                     double *wpart, hipStream_t s) {
+    hipLaunchKernelGGL(k_b_bicg_p, dim3(m.nblk), dim3(BS), 0, s, op, tab, m, p, r, AMp, wpart);
     CUIBM_LAUNCH_CHECK();
 }
 

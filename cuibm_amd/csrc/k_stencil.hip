@@ -697,26 +697,8 @@ __global__ void __launch_bounds__(BS) k_b_wdot(const BCase *__restrict__ tab, BM
     if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
 }
 
-__global__ void __launch_bounds__(BS) k_b_wdot_finish(const BCase *__restrict__ tab, const int *__restrict__ first,
-                                                      const double *__restrict__ part,
-                                                      const double *__restrict__ inv_wa, double *__restrict__ defl) {
-    const int c = blockIdx.x;
-    const BCase &C = tab[c];
-    if (C.p5.stop && *C.p5.stop != 0.0) return;  // uniform per block
-    double acc[1] = {0};
-    for (int k = first[c] + (int)threadIdx.x; k < first[c + 1]; k += BS) acc[0] += part[k];
-    block_sum<1>(acc);
-    if (threadIdx.x == 0) defl[c] = acc[0] * inv_wa[c];
-}
-
 void launch_b_wdot(const BCase *tab, const BMapDev &m, const double *r, double *part, hipStream_t s) {
     hipLaunchKernelGGL(k_b_wdot, dim3(m.nblk), dim3(BS), 0, s, tab, m, r, part);
-    CUIBM_LAUNCH_CHECK();
-}
-
-void launch_b_wdot_finish(const BCase *tab, int ncases, const int *first, const double *part, const double *inv_wa,
-                          double *defl, hipStream_t s) {
-    hipLaunchKernelGGL(k_b_wdot_finish, dim3(ncases), dim3(BS), 0, s, tab, first, part, inv_wa, defl);
     CUIBM_LAUNCH_CHECK();
 }
 

@@ -782,9 +782,10 @@ struct BatchMg::Impl {
         BMap tiles[2];
         std::vector<long> nt[2];
 
-        void add(const TensorMg::Levels<T> &C, long off, const double *stop, double *c) {
+        void add(const TensorMg::Levels<T> &C, long off, const double *stop, double *c, const double *part, int npart) {
             auto pins = [&](MgPins P) {
-                P.part = nullptr;  // the batch forms each case's constant
+                P.part = part;
+                P.npart = npart;
                 P.c = c;
                 return P;
             };
@@ -858,49 +859,41 @@ struct BatchMg::Impl {
     };
     Set<double> d;
     Set<float> f;
-    const BCase *tab = nullptr;
-    BMapDev pmap{};
-    const int *pfirst = nullptr;
-    int ncases = 0, levels = 0;
-    DArray<double> part, inv_wa, c;
+    int levels = 0;
+    DArray<double> part, c;
 };
 
-BatchMg::BatchMg(const std::vector<TensorMg *> &mg, const std::vector<long> &offP, const BCase *tab_dev,
-                 const std::vector<BCase> &tab_host, const BMapDev &pmap, const int *pfirst, hipStream_t s)
+BatchMg::BatchMg(const std::vector<TensorMg *> &mg, const std::vector<long> &offP, const std::vector<BCase> &tab_host,
+                 const std::vector<int> &nblk, hipStream_t s)
     : im_(new Impl) {
     if (mg.empty()) throw Error("batched V-cycle without cases", ERR_ARGUMENT);
     Impl &B = *im_;
-    B.ncases = (int)mg.size();
-    B.tab = tab_dev;
-    B.pmap = pmap;
-    B.pfirst = pfirst;
     B.c.alloc(mg.size());
     launch_fill(B.c.p(), 0.0, (long)mg.size(), s);
-    std::vector<double> iw;
+    size_t total = 0, first = 0;
+    for (int n : nblk) total += n;
+    B.part.alloc(std::max<size_t>(total, 1));
     for (size_t k = 0; k < mg.size(); k++) {
         const TensorMg &M = *mg[k];
         const double *stop = tab_host[k].scP + SC_STOP;
-        double *c = B.c.p() + k;
         auto take = [&](auto &set, const auto &L) {
-            iw.push_back(L.fine_direct ? L.direct.pins.inv_wa : L.lv[0].task.pins.inv_wa);
-            set.add(L, offP[k], stop, c);
+            set.add(L, offP[k], stop, B.c.p() + k, B.part.p() + first, nblk[k]);
         };
         if (M.f_) take(B.f, *M.f_);
         else take(B.d, *M.d_);
+        first += nblk[k];
         B.levels = std::max(B.levels, (int)M.sizes().size());
     }
-    B.inv_wa.upload(iw, s);
-    B.part.alloc(std::max(pmap.nblk, 1));
     B.d.finish(s);
     B.f.finish(s);
 }
+
+double *BatchMg::weights_part() const { return im_->part.p(); }
 
 BatchMg::~BatchMg() = default;
 
 void BatchMg::apply(const double *r, double *z, hipStream_t s) {
     Impl &B = *im_;
-    launch_b_wdot(B.tab, B.pmap, r, B.part.p(), s);
-    launch_b_wdot_finish(B.tab, B.ncases, B.pfirst, B.part.p(), B.inv_wa.p(), B.c.p(), s);
     B.d.apply(r, z, s);
     B.f.apply(r, z, s);
 }
