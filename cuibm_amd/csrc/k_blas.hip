@@ -1,6 +1,6 @@
 // Vector, reduction and sparse-product kernels for the Krylov and AMG solvers.
 //
-// Reductions are deterministic: a grid that depends on n alone (red_blocks) strides over the
+// Reductions are deterministic: groups that depend on n alone (red_parts) strides over the
 // vector, each block reduces its threads in a fixed tree (wavefront shuffles, then
 // LDS across the 4 wavefronts of a 256-thread block) and writes one partial; the
 // consumer, or a single-block kernel, then sums the partials in a fixed order. The result
@@ -94,28 +94,31 @@ template void launch_spmv<float, double>(const DCsr<float> &, const double *, do
 // at every gather, and written to Mp.
 // Each block takes a contiguous chunk of rows, and the chunks of one XCD are contiguous too, so
 // that the gathers of x from neighbouring rows stay in that XCD's L2.
-template <bool JAC>
-__global__ void __launch_bounds__(BS) k_spmv_dot(int n, const int *__restrict__ rp, const int *__restrict__ ci,
-                                                 const double *__restrict__ v, const double *__restrict__ x,
+template <bool JAC, int TB>
+__global__ void __launch_bounds__(TB) k_spmv_dot(int n, const int *__restrict__ rp, const int *__restrict__ ci,
+                                                 const double *__restrict__ val, const double *__restrict__ x,
                                                  const double *__restrict__ dinv, double *__restrict__ Mp,
                                                  double *__restrict__ y, const double *__restrict__ a, int want_yy,
                                                  FinArgs f, double *__restrict__ part, const double *__restrict__ stop) {
     const double stopv = stop ? *stop : 0.0;  // read at once, tested after the first row
     if (JAC && f.part) {
         double tot[2] = {0, 0};
-        finish_sums<1>(f, tot);
+        finish_sums<1, TB>(f, tot);
         if (stopv != 0.0) return;  // uniform, as every return before the last barrier
         if (fin_ss(tot, f.sc, blockIdx.x == 0 && threadIdx.x == 0) != 0.0) return;
     }
     double acc[2] = {0, 0};
     bool tested = false;
-    const int nb = gridDim.x, chunk = (n + nb - 1) / nb, r0 = xcd_block(nb) * chunk, r1 = min(n, r0 + chunk);
-    for (int i = r0 + threadIdx.x; i < r1; i += BS) {
+    const int np = red_parts(n), chunk = (n + np - 1) / np;
+    // group v = x + 8 c takes chunk x np / 8 + c; the groups of a block share x, its XCD
+    const int c = red_group<TB>(blockIdx.x / 8), v = c < np / 8 ? (int)(blockIdx.x % 8) + 8 * c : np;
+    const int r0 = v < np ? ((int)(blockIdx.x % 8) * (np / 8) + c) * chunk : n, r1 = min(n, r0 + chunk);
+    for (int i = r0 + red_lane(); i < r1; i += BS) {
         double yi;
         if (JAC) {
-            yi = csr_lane_sum<double, 1>(ci, v, rp[i], rp[i + 1], [&](int c) { return dinv[c] * x[c]; });
+            yi = csr_lane_sum<double, 1>(ci, val, rp[i], rp[i + 1], [&](int c) { return dinv[c] * x[c]; });
         } else {
-            yi = row_dot(rp, ci, v, x, i);
+            yi = row_dot(rp, ci, val, x, i);
         }
         if (!tested) {
             if (stopv != 0.0) return;  // every thread returns here or below: no barrier is reached
@@ -127,124 +130,126 @@ __global__ void __launch_bounds__(BS) k_spmv_dot(int n, const int *__restrict__ 
         acc[1] += yi * yi;
     }
     if (stopv != 0.0) return;
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = acc[0];
-        if (want_yy) part[RED_GRID + blockIdx.x] = acc[1];
+    block_sum<2, TB>(acc);
+    if (red_lane() == 0 && v < np) {
+        part[v] = acc[0];
+        if (want_yy) part[np + v] = acc[1];
     }
 }
 
 void launch_spmv_dot(const DCsr<double> &A, const double *x, double *y, const double *a, bool want_yy, double *part,
                      hipStream_t s, const double *stop) {
-    hipLaunchKernelGGL(k_spmv_dot<false>, dim3(red_blocks(A.n)), dim3(BS), 0, s, A.n, A.rp.p(), A.ci.p(), A.v.p(), x,
-                       nullptr, nullptr, y, a, (int)want_yy, FinArgs{}, part, stop);
+    by_block(A.n, [&](auto tb) {
+        hipLaunchKernelGGL((k_spmv_dot<false, tb>), dim3(red_grid(A.n)), dim3(tb), 0, s, A.n, A.rp.p(), A.ci.p(),
+                           A.v.p(), x, nullptr, nullptr, y, a, (int)want_yy, FinArgs{}, part, stop);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
 void launch_spmv_dot_jacobi(const DCsr<double> &A, const double *dinv, const double *p, double *Mp, double *y,
                             const double *a, bool want_yy, const FinArgs &f, double *part, hipStream_t s,
                             const double *stop) {
-    hipLaunchKernelGGL(k_spmv_dot<true>, dim3(red_blocks(A.n)), dim3(BS), 0, s, A.n, A.rp.p(), A.ci.p(), A.v.p(), p,
-                       dinv, Mp, y, a, (int)want_yy, f, part, stop);
+    by_block(A.n, [&](auto tb) {
+        hipLaunchKernelGGL((k_spmv_dot<true, tb>), dim3(red_grid(A.n)), dim3(tb), 0, s, A.n, A.rp.p(), A.ci.p(),
+                           A.v.p(), p, dinv, Mp, y, a, (int)want_yy, f, part, stop);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
 // r = b - A x; also p = r and rs = r when given; partials of (r.r) and (b.b)
-__global__ void __launch_bounds__(BS) k_bicg_init(int n, const int *__restrict__ rp, const int *__restrict__ ci,
-                                                  const double *__restrict__ v, const double *__restrict__ x,
+template <int TB>
+__global__ void __launch_bounds__(TB) k_bicg_init(int n, const int *__restrict__ rp, const int *__restrict__ ci,
+                                                  const double *__restrict__ val, const double *__restrict__ x,
                                                   const double *__restrict__ b, double *__restrict__ r,
                                                   double *__restrict__ p, double *__restrict__ rs,
                                                   double *__restrict__ part) {
     double acc[2] = {0, 0};
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const int np = red_parts(n), v = red_group<TB>(blockIdx.x);
+    for (int i = v < np ? v * BS + red_lane() : n; i < n; i += np * BS) {
         const double bi = b[i];
-        const double ri = bi - row_dot(rp, ci, v, x, i);
+        const double ri = bi - row_dot(rp, ci, val, x, i);
         r[i] = ri;
         p[i] = ri;
         rs[i] = ri;
         acc[0] += ri * ri;
         acc[1] += bi * bi;
     }
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = acc[0];
-        part[RED_GRID + blockIdx.x] = acc[1];
+    block_sum<2, TB>(acc);
+    if (red_lane() == 0 && v < np) {
+        part[v] = acc[0];
+        part[np + v] = acc[1];
     }
 }
 
 void launch_bicg_init(const DCsr<double> &A, const double *x, const double *b, double *r, double *p, double *rs,
                       double *part, hipStream_t s) {
-    hipLaunchKernelGGL(k_bicg_init, dim3(red_blocks(A.n)), dim3(BS), 0, s, A.n, A.rp.p(), A.ci.p(), A.v.p(), x, b, r, p, rs,
-                       part);
+    by_block(A.n, [&](auto tb) {
+        hipLaunchKernelGGL(k_bicg_init<tb>, dim3(red_grid(A.n)), dim3(tb), 0, s, A.n, A.rp.p(), A.ci.p(), A.v.p(), x,
+                           b, r, p, rs, part);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
 // s = r - alpha AMp with partials of (s.s)
-template <bool W>
-__global__ void __launch_bounds__(BS) k_bicg_s(int n, const double *__restrict__ r, const double *__restrict__ AMp,
+template <bool W, int TB>
+__global__ void __launch_bounds__(TB) k_bicg_s(int n, const double *__restrict__ r, const double *__restrict__ AMp,
                                                double *__restrict__ s, FinArgs f, double *__restrict__ part,
                                                InputWeights w) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int np = red_parts(n), v = red_group<TB>(blockIdx.x);
+    int i = v < np ? v * BS + red_lane() : n;
     double rv = i < n ? r[i] : 0.0, av = i < n ? AMp[i] : 0.0;  // in flight during the finish
     const double stopv = f.sc[sc_stop(f.par)];
-    double alpha;
-    if (f.part) {
-        double tot[2] = {0, 0};
-        finish_sums<1>(f, tot);
-        if (stopv != 0.0) return;  // uniform, as every return before the last barrier
-        alpha = fin_alpha(tot, f.sc, f.par, blockIdx.x == 0 && threadIdx.x == 0);
-    } else {
-        alpha = f.sc[SC_ALPHA];
-    }
-    if (stopv != 0.0) return;
+    double tot[2] = {0, 0};
+    finish_sums<1, TB>(f, tot);
+    if (stopv != 0.0) return;  // uniform, as every return before the last barrier
+    const double alpha = fin_alpha(tot, f.sc, f.par, blockIdx.x == 0 && threadIdx.x == 0);
     double acc[2] = {0, 0};
     while (i < n) {
         const double si = rv - alpha * av;
         s[i] = si;
         acc[0] += si * si;
         if (W) acc[1] += (w.wx[i % w.nx] * w.wy[i / w.nx]) * si;
-        i += gridDim.x * blockDim.x;
+        i += np * BS;
         if (i < n) {
             rv = r[i];
             av = AMp[i];
         }
     }
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = acc[0];
-        if (W) w.part[blockIdx.x] = acc[1];
+    block_sum<2, TB>(acc);
+    if (red_lane() == 0 && v < np) {
+        part[v] = acc[0];
+        if (W) w.part[v] = acc[1];
     }
 }
 
 void launch_bicg_s(int n, const double *r, const double *AMp, double *s_, const FinArgs &f, double *part,
                    hipStream_t s, const InputWeights *w) {
-    const dim3 g(red_blocks(n));
-    if (w) hipLaunchKernelGGL(k_bicg_s<true>, g, dim3(BS), 0, s, n, r, AMp, s_, f, part, *w);
-    else hipLaunchKernelGGL(k_bicg_s<false>, g, dim3(BS), 0, s, n, r, AMp, s_, f, part, InputWeights{});
+    const dim3 g(red_grid(n));
+    by_block(n, [&](auto tb) {
+        if (w) hipLaunchKernelGGL((k_bicg_s<true, tb>), g, dim3(tb), 0, s, n, r, AMp, s_, f, part, *w);
+        else hipLaunchKernelGGL((k_bicg_s<false, tb>), g, dim3(tb), 0, s, n, r, AMp, s_, f, part, InputWeights{});
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
 // x += alpha Mp + omega Ms; r = s - omega AMs; partials of (rs.r) and (r.r). In the
 // iteration that ended at its half step (STOP_HALF_PENDING) it applies the half-step update
 // x += alpha Mp alone.
-__global__ void __launch_bounds__(BS) k_bicg_xr(int n, double *__restrict__ x, const double *__restrict__ Mp,
+template <int TB>
+__global__ void __launch_bounds__(TB) k_bicg_xr(int n, double *__restrict__ x, const double *__restrict__ Mp,
                                                 const double *__restrict__ Ms, double *__restrict__ r,
                                                 const double *__restrict__ s, const double *__restrict__ AMs,
                                                 const double *__restrict__ rs, FinArgs f, double *__restrict__ part) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int np = red_parts(n), v = red_group<TB>(blockIdx.x);
+    int i = v < np ? v * BS + red_lane() : n;
     auto at = [&](const double *a) { return i < n ? a[i] : 0.0; };
     double xv = at(x), mp = at(Mp), ms = at(Ms), sv = at(s), am = at(AMs), rv = at(rs);  // in flight during the finish
     const double stopv = f.sc[sc_stop(f.par)], half_code = f.sc[SC_STOPS], alpha = f.sc[SC_ALPHA];
     const bool half = stopv == 0.0 && half_code == STOP_HALF_PENDING;
     const bool stopped = stopv != 0.0 || half_code != 0.0;
-    double omega = 0;
-    if (f.part) {
-        double tot[2] = {0, 0};
-        finish_sums<2>(f, tot);
-        if (!stopped) omega = fin_omega(tot, f.sc, blockIdx.x == 0 && threadIdx.x == 0);
-    } else {
-        omega = f.sc[SC_OMEGA];
-    }
+    double tot[2] = {0, 0};
+    finish_sums<2, TB>(f, tot);
+    const double omega = stopped ? 0.0 : fin_omega(tot, f.sc, blockIdx.x == 0 && threadIdx.x == 0);
     if (stopped && !half) return;  // uniform, as every return before the last barrier
     double acc[2] = {0, 0};
     while (i < n) {
@@ -258,7 +263,7 @@ __global__ void __launch_bounds__(BS) k_bicg_xr(int n, double *__restrict__ x, c
             acc[0] += rv * ri;
             acc[1] += ri * ri;
         }
-        i += gridDim.x * blockDim.x;
+        i += np * BS;
         if (i < n) {
             xv = x[i];
             mp = Mp[i];
@@ -269,47 +274,44 @@ __global__ void __launch_bounds__(BS) k_bicg_xr(int n, double *__restrict__ x, c
         }
     }
     if (half) return;
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = acc[0];
-        part[RED_GRID + blockIdx.x] = acc[1];
+    block_sum<2, TB>(acc);
+    if (red_lane() == 0 && v < np) {
+        part[v] = acc[0];
+        part[np + v] = acc[1];
     }
 }
 
 void launch_bicg_xr(int n, double *x, const double *Mp, const double *Ms, double *r, const double *s_,
                     const double *AMs, const double *rs, const FinArgs &f, double *part, hipStream_t s) {
-    hipLaunchKernelGGL(k_bicg_xr, dim3(red_blocks(n)), dim3(BS), 0, s, n, x, Mp, Ms, r, s_, AMs, rs, f, part);
+    by_block(n, [&](auto tb) {
+        hipLaunchKernelGGL(k_bicg_xr<tb>, dim3(red_grid(n)), dim3(tb), 0, s, n, x, Mp, Ms, r, s_, AMs, rs, f, part);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
 // p = r + beta p - beta omega AMp; W: with the weighted partial sums of the new p
-template <bool W>
-__global__ void __launch_bounds__(BS) k_bicg_p(int n, double *__restrict__ p, const double *__restrict__ r,
+template <bool W, int TB>
+__global__ void __launch_bounds__(TB) k_bicg_p(int n, double *__restrict__ p, const double *__restrict__ r,
                                                const double *__restrict__ AMp, FinArgs f, InputWeights w) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int np = red_parts(n), v = red_group<TB>(blockIdx.x);
+    int i = v < np ? v * BS + red_lane() : n;
     double pv = i < n ? p[i] : 0.0, rv = i < n ? r[i] : 0.0, av = i < n ? AMp[i] : 0.0;  // in flight during the finish
     const double omega = f.sc[SC_OMEGA];
-    double beta;
-    if (f.part) {
-        const bool one = blockIdx.x == 0 && threadIdx.x == 0;
-        const bool stopped = f.sc[sc_stop(f.par)] != 0.0 || f.sc[SC_STOPS] != 0.0;
-        double tot[2] = {0, 0};
-        finish_sums<2>(f, tot);
-        if (stopped) {
-            if (one) pass_stop(f.sc, f.par);
-            return;  // uniform, as every return before the last barrier
-        }
-        beta = fin_beta(tot, f.sc, f.par, f.maxit, one);  // a p past the last iteration is not used
-    } else {
-        if (f.sc[sc_stop(f.par ^ 1)] != 0.0) return;
-        beta = f.sc[SC_BETA];
+    const bool one = blockIdx.x == 0 && threadIdx.x == 0;
+    const bool stopped = f.sc[sc_stop(f.par)] != 0.0 || f.sc[SC_STOPS] != 0.0;
+    double tot[2] = {0, 0};
+    finish_sums<2, TB>(f, tot);
+    if (stopped) {
+        if (one) pass_stop(f.sc, f.par);
+        return;  // uniform, as every return before the last barrier
     }
+    const double beta = fin_beta(tot, f.sc, f.par, f.maxit, one);  // a p past the last iteration is not used
     double acc[1] = {0};
     while (i < n) {
-        const double v = rv + beta * pv - beta * omega * av;
-        p[i] = v;
-        if (W) acc[0] += (w.wx[i % w.nx] * w.wy[i / w.nx]) * v;
-        i += gridDim.x * blockDim.x;
+        const double pi = rv + beta * pv - beta * omega * av;
+        p[i] = pi;
+        if (W) acc[0] += (w.wx[i % w.nx] * w.wy[i / w.nx]) * pi;
+        i += np * BS;
         if (i < n) {
             pv = p[i];
             rv = r[i];
@@ -317,15 +319,17 @@ __global__ void __launch_bounds__(BS) k_bicg_p(int n, double *__restrict__ p, co
         }
     }
     if (!W) return;
-    block_sum<1>(acc);
-    if (threadIdx.x == 0) w.part[blockIdx.x] = acc[0];
+    block_sum<1, TB>(acc);
+    if (red_lane() == 0 && v < np) w.part[v] = acc[0];
 }
 
 void launch_bicg_p(int n, double *p, const double *r, const double *AMp, const FinArgs &f, hipStream_t s,
                    const InputWeights *w) {
-    const dim3 g(red_blocks(n));
-    if (w) hipLaunchKernelGGL(k_bicg_p<true>, g, dim3(BS), 0, s, n, p, r, AMp, f, *w);
-    else hipLaunchKernelGGL(k_bicg_p<false>, g, dim3(BS), 0, s, n, p, r, AMp, f, InputWeights{});
+    const dim3 g(red_grid(n));
+    by_block(n, [&](auto tb) {
+        if (w) hipLaunchKernelGGL((k_bicg_p<true, tb>), g, dim3(tb), 0, s, n, p, r, AMp, f, *w);
+        else hipLaunchKernelGGL((k_bicg_p<false, tb>), g, dim3(tb), 0, s, n, p, r, AMp, f, InputWeights{});
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
@@ -374,66 +378,34 @@ __device__ __forceinline__ void finish_update(int op, const double (&tot)[2], do
     }
 }
 
-// sum the partial groups and update the recurrence scalars (one block)
-__global__ void __launch_bounds__(1024) k_bicg_finish(const double *__restrict__ part, int np, int op, FinArgs f,
-                                                      double rtol) {
+// sum the partial groups and update the recurrence scalars (one block): of a (re)start, or, where
+// the next launches have to know whether the half step ended the solve, FIN_SS
+__global__ void __launch_bounds__(1024) k_bicg_finish(int op, FinArgs f, double rtol) {
     double *sc = f.sc;
-    const bool start = op == FIN_INIT || op == FIN_RESTART;
-    // the codes that stop this finish, tested after the loads
-    const double stopv = start ? 0.0 : sc[sc_stop(f.par)];
-    const double half = start || op == FIN_ALPHA || op == FIN_SS ? 0.0 : sc[SC_STOPS];
-    __shared__ double sh[2][16];
-    double v[2] = {0, 0};
-    const int ng = (op == FIN_ALPHA || op == FIN_SS) ? 1 : 2;
-    for (int g = 0; g < ng; g++) {
-        double t = 0;
-        for (int k = threadIdx.x; k < np; k += blockDim.x) t += part[g * RED_GRID + k];
-        v[g] = t;
-    }
-    if (stopv != 0.0 || half != 0.0) {  // uniform across the block, before the barrier
-        if (threadIdx.x == 0) {
-            if (op == FIN_SS) sc[SC_STOPS] = stopv;  // what the second half reads
-            if (op == FIN_BETA) pass_stop(sc, f.par);
-        }
+    const double stopv = op == FIN_SS ? sc[sc_stop(f.par)] : 0.0;
+    double tot[2] = {0, 0};
+    finish_sums<2, 1024>(f, tot);
+    if (threadIdx.x != 0) return;
+    if (op == FIN_SS) {
+        if (stopv != 0.0) sc[SC_STOPS] = stopv;  // what the second half reads
+        else fin_ss(tot, sc, true);
         return;
     }
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    for (int g = 0; g < ng; g++) {
-        double t = wave_sum(v[g]);
-        if (lane == 0) sh[g][wid] = t;
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    double tot[2] = {0, 0};
-    for (int g = 0; g < ng; g++) {
-        double t = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); w++) t += sh[g][w];
-        tot[g] = t;
-    }
-    switch (op) {
-        case FIN_INIT:  // (r.r, b.b)
-        case FIN_RESTART:
-            sc[SC_RR] = tot[0];
-            sc[SC_RHO] = tot[0];
-            sc[SC_STOPS] = 0.0;
-            sc[SC_STOP] = 0.0;
-            if (op == FIN_INIT) {
-                sc[SC_BB] = tot[1];
-                sc[SC_D0] = tot[0];
-                sc[SC_ITS] = 0.0;
-                sc[SC_TOL] = rtol * sqrt(tot[1]);
-                if (sqrt(tot[0]) <= sc[SC_TOL]) sc[SC_STOP] = STOP_CONVERGED;
-            }
-            break;
-        case FIN_ALPHA: fin_alpha(tot, sc, f.par, true); break;
-        case FIN_SS: fin_ss(tot, sc, true); break;
-        case FIN_OMEGA: fin_omega(tot, sc, true); break;
-        case FIN_BETA: fin_beta(tot, sc, f.par, f.maxit, true); break;
+    sc[SC_RR] = tot[0];  // (r.r, b.b)
+    sc[SC_RHO] = tot[0];
+    sc[SC_STOPS] = 0.0;
+    sc[SC_STOP] = 0.0;
+    if (op == FIN_INIT) {
+        sc[SC_BB] = tot[1];
+        sc[SC_D0] = tot[0];
+        sc[SC_ITS] = 0.0;
+        sc[SC_TOL] = rtol * sqrt(tot[1]);
+        if (sqrt(tot[0]) <= sc[SC_TOL]) sc[SC_STOP] = STOP_CONVERGED;
     }
 }
 
-void launch_bicg_finish(const double *part, int np, int op, const FinArgs &f, hipStream_t s, double rtol) {
-    hipLaunchKernelGGL(k_bicg_finish, dim3(1), dim3(1024), 0, s, part, np, op, f, rtol);
+void launch_bicg_finish(int op, const FinArgs &f, hipStream_t s, double rtol) {
+    hipLaunchKernelGGL(k_bicg_finish, dim3(1), dim3(1024), 0, s, op, f, rtol);
     CUIBM_LAUNCH_CHECK();
 }
 

@@ -64,22 +64,22 @@ __global__ void k_p5_coef(int nx, int ny, const double *__restrict__ dx, const d
 
 // y = A x with partials of (y . a) and (y . y). JAC: x = D^-1 p, formed at every point of the row,
 // and written to Mp (as the CSR k_spmv_dot).
-template <bool JAC>
-__global__ void __launch_bounds__(BS) k_p5_spmv_dot(P5Dev A, const double *__restrict__ x,
+template <bool JAC, int TB>
+__global__ void __launch_bounds__(TB) k_p5_spmv_dot(P5Dev A, const double *__restrict__ x,
                                                     const double *__restrict__ dinv, double *__restrict__ Mp,
                                                     double *__restrict__ y, const double *__restrict__ a, int want_yy,
                                                     FinArgs f, double *__restrict__ part) {
     const double stopv = A.stop ? *A.stop : 0.0;  // the Krylov solve's stop code, tested after the loads
     if (JAC && f.part) {
         double tot[2] = {0, 0};
-        finish_sums<1>(f, tot);
+        finish_sums<1, TB>(f, tot);
         if (stopv != 0.0) return;  // uniform, as every return before the last barrier
         if (fin_ss(tot, f.sc, blockIdx.x == 0 && threadIdx.x == 0) != 0.0) return;
     }
-    const int n = A.nx * A.ny, nb = gridDim.x, blk = xcd_band(nb);
+    const int n = A.nx * A.ny, np = red_parts(n), v = red_group<TB>(xcd_band(gridDim.x));
     double acc[2] = {0, 0};
     bool tested = false;
-    for (int ip = blk * BS + threadIdx.x; ip < n; ip += nb * BS) {
+    for (int ip = v < np ? v * BS + red_lane() : n; ip < n; ip += np * BS) {
         const int I = ip % A.nx, J = ip / A.nx;
         const double yi = p5_row(
             A, I, J, p5_diag(A, I, J, ip), [&](int o) { return JAC ? dinv[ip + o] * x[ip + o] : x[ip + o]; }, A.nx);
@@ -93,20 +93,21 @@ __global__ void __launch_bounds__(BS) k_p5_spmv_dot(P5Dev A, const double *__res
         acc[1] += yi * yi;
     }
     if (stopv != 0.0) return;
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[blk] = acc[0];
-        if (want_yy) part[RED_GRID + blk] = acc[1];
+    block_sum<2, TB>(acc);
+    if (red_lane() == 0 && v < np) {
+        part[v] = acc[0];
+        if (want_yy) part[np + v] = acc[1];
     }
 }
 
 // r = b - A x, p = rs = r, partials of (r . r) and (b . b)
-__global__ void __launch_bounds__(BS) k_p5_init(P5Dev A, const double *__restrict__ x, const double *__restrict__ b,
+template <int TB>
+__global__ void __launch_bounds__(TB) k_p5_init(P5Dev A, const double *__restrict__ x, const double *__restrict__ b,
                                                 double *__restrict__ r, double *__restrict__ p,
                                                 double *__restrict__ rs, double *__restrict__ part) {
-    const int n = A.nx * A.ny, blk = xcd_band(gridDim.x);
+    const int n = A.nx * A.ny, np = red_parts(n), v = red_group<TB>(xcd_band(gridDim.x));
     double acc[2] = {0, 0};
-    for (int ip = blk * BS + threadIdx.x; ip < n; ip += gridDim.x * BS) {
+    for (int ip = v < np ? v * BS + red_lane() : n; ip < n; ip += np * BS) {
         const int I = ip % A.nx, J = ip / A.nx;
         const double bi = b[ip];
         const double ri = bi - p5_row(A, I, J, p5_diag(A, I, J, ip), [&](int o) { return x[ip + o]; }, A.nx);
@@ -116,10 +117,10 @@ __global__ void __launch_bounds__(BS) k_p5_init(P5Dev A, const double *__restric
         acc[0] += ri * ri;
         acc[1] += bi * bi;
     }
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[blk] = acc[0];
-        part[RED_GRID + blk] = acc[1];
+    block_sum<2, TB>(acc);
+    if (red_lane() == 0 && v < np) {
+        part[v] = acc[0];
+        part[np + v] = acc[1];
     }
 }
 
@@ -331,15 +332,16 @@ __global__ void __launch_bounds__(256) k_p5_sweep2(P5Dev A, double w, const doub
 }
 
 // partial sums of w_i r_i, w_i = dx[I] dy[J]
-__global__ void __launch_bounds__(BS) k_p5_wdot(P5Dev A, const double *__restrict__ r, double *__restrict__ part) {
+template <int TB>
+__global__ void __launch_bounds__(TB) k_p5_wdot(P5Dev A, const double *__restrict__ r, double *__restrict__ part) {
     const double stopv = A.stop ? *A.stop : 0.0;
     if (stopv != 0.0) return;
-    const int n = A.nx * A.ny, blk = xcd_band(gridDim.x);
+    const int n = A.nx * A.ny, np = red_parts(n), v = red_group<TB>(xcd_band(gridDim.x));
     double acc[1] = {0};
-    for (int ip = blk * BS + threadIdx.x; ip < n; ip += gridDim.x * BS)
+    for (int ip = v < np ? v * BS + red_lane() : n; ip < n; ip += np * BS)
         acc[0] += (A.dx[ip % A.nx] * A.dy[ip / A.nx]) * r[ip];
-    block_sum<1>(acc);
-    if (threadIdx.x == 0) part[blk] = acc[0];
+    block_sum<1, TB>(acc);
+    if (red_lane() == 0 && v < np) part[v] = acc[0];
 }
 
 // one sweep xn = x + omega D^-1 (b - A x), a row per thread
@@ -386,21 +388,27 @@ PoissonStencil::PoissonStencil(const GridDev &g, double dt, bool centre_pin, hip
 
 void PoissonStencil::spmv_dot(const double *x, double *y, const double *a, bool want_yy, double *part,
                               hipStream_t s) const {
-    hipLaunchKernelGGL(k_p5_spmv_dot<false>, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), x, nullptr, nullptr, y, a,
-                       (int)want_yy, FinArgs{}, part);
+    by_block(n(), [&](auto tb) {
+        hipLaunchKernelGGL((k_p5_spmv_dot<false, tb>), dim3(red_grid(n())), dim3(tb), 0, s,
+                           dev(), x, nullptr, nullptr, y, a, (int)want_yy, FinArgs{}, part);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
 void PoissonStencil::spmv_dot_jacobi(const double *dinv, const double *p, double *Mp, double *y, const double *a,
                                      bool want_yy, const FinArgs &f, double *part, hipStream_t s) const {
-    hipLaunchKernelGGL(k_p5_spmv_dot<true>, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), p, dinv, Mp, y, a,
-                       (int)want_yy, f, part);
+    by_block(n(), [&](auto tb) {
+        hipLaunchKernelGGL((k_p5_spmv_dot<true, tb>), dim3(red_grid(n())), dim3(tb), 0, s,
+                           dev(), p, dinv, Mp, y, a, (int)want_yy, f, part);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
 void PoissonStencil::init(const double *x, const double *b, double *r, double *p, double *rs, double *part,
                           hipStream_t s) const {
-    hipLaunchKernelGGL(k_p5_init, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), x, b, r, p, rs, part);
+    by_block(n(), [&](auto tb) {
+        hipLaunchKernelGGL(k_p5_init<tb>, dim3(red_grid(n())), dim3(tb), 0, s, dev(), x, b, r, p, rs, part);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
@@ -471,21 +479,22 @@ __device__ __forceinline__ double v5_row(const V5Dev &A, int i, F x) {
 }
 
 // y = A x with block partials of (y . a) and (y . y); JAC as in k_p5_spmv_dot
-template <bool JAC>
-__global__ void __launch_bounds__(BS) k_v5_spmv_dot(V5Dev A, int n, const double *__restrict__ x,
+template <bool JAC, int TB>
+__global__ void __launch_bounds__(TB) k_v5_spmv_dot(V5Dev A, int n, const double *__restrict__ x,
                                                     const double *__restrict__ dinv, double *__restrict__ Mp,
                                                     double *__restrict__ y, const double *__restrict__ a, int want_yy,
                                                     FinArgs f, double *__restrict__ part) {
     const double stopv = A.stop ? *A.stop : 0.0;  // the Krylov solve's stop code, tested after the loads
     if (JAC && f.part) {
         double tot[2] = {0, 0};
-        finish_sums<1>(f, tot);
+        finish_sums<1, TB>(f, tot);
         if (stopv != 0.0) return;  // uniform, as every return before the last barrier
         if (fin_ss(tot, f.sc, blockIdx.x == 0 && threadIdx.x == 0) != 0.0) return;
     }
     double acc[2] = {0, 0};
     bool tested = false;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const int np = red_parts(n), v = red_group<TB>(blockIdx.x);
+    for (int i = v < np ? v * BS + red_lane() : n; i < n; i += np * BS) {
         const double yi = v5_row(A, i, [&](int j) { return JAC ? dinv[j] * x[j] : x[j]; });
         if (!tested) {
             if (stopv != 0.0) return;  // every thread returns here or below: no barrier is reached
@@ -497,20 +506,22 @@ __global__ void __launch_bounds__(BS) k_v5_spmv_dot(V5Dev A, int n, const double
         acc[1] += yi * yi;
     }
     if (stopv != 0.0) return;
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = acc[0];
-        if (want_yy) part[RED_GRID + blockIdx.x] = acc[1];
+    block_sum<2, TB>(acc);
+    if (red_lane() == 0 && v < np) {
+        part[v] = acc[0];
+        if (want_yy) part[np + v] = acc[1];
     }
 }
 
 // r = b - A x, p = rs = r, partials of (r . r) and (b . b): as the CSR k_bicg_init
-__global__ void __launch_bounds__(BS) k_v5_init(V5Dev A, int n, const double *__restrict__ x,
+template <int TB>
+__global__ void __launch_bounds__(TB) k_v5_init(V5Dev A, int n, const double *__restrict__ x,
                                                 const double *__restrict__ b, double *__restrict__ r,
                                                 double *__restrict__ p, double *__restrict__ rs,
                                                 double *__restrict__ part) {
     double acc[2] = {0, 0};
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const int np = red_parts(n), v = red_group<TB>(blockIdx.x);
+    for (int i = v < np ? v * BS + red_lane() : n; i < n; i += np * BS) {
         const double bi = b[i];
         const double ri = bi - v5_row(A, i, [&](int j) { return x[j]; });
         r[i] = ri;
@@ -519,10 +530,10 @@ __global__ void __launch_bounds__(BS) k_v5_init(V5Dev A, int n, const double *__
         acc[0] += ri * ri;
         acc[1] += bi * bi;
     }
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = acc[0];
-        part[RED_GRID + blockIdx.x] = acc[1];
+    block_sum<2, TB>(acc);
+    if (red_lane() == 0 && v < np) {
+        part[v] = acc[0];
+        part[np + v] = acc[1];
     }
 }
 
@@ -547,21 +558,27 @@ V5Dev VelocityStencil::dev() const {
 
 void VelocityStencil::spmv_dot(const double *x, double *y, const double *a, bool want_yy, double *part,
                                hipStream_t s) const {
-    hipLaunchKernelGGL(k_v5_spmv_dot<false>, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), n(), x, nullptr, nullptr, y,
-                       a, (int)want_yy, FinArgs{}, part);
+    by_block(n(), [&](auto tb) {
+        hipLaunchKernelGGL((k_v5_spmv_dot<false, tb>), dim3(red_grid(n())), dim3(tb), 0, s,
+                           dev(), n(), x, nullptr, nullptr, y, a, (int)want_yy, FinArgs{}, part);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
 void VelocityStencil::spmv_dot_jacobi(const double *dinv, const double *p, double *Mp, double *y, const double *a,
                                       bool want_yy, const FinArgs &f, double *part, hipStream_t s) const {
-    hipLaunchKernelGGL(k_v5_spmv_dot<true>, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), n(), p, dinv, Mp, y, a,
-                       (int)want_yy, f, part);
+    by_block(n(), [&](auto tb) {
+        hipLaunchKernelGGL((k_v5_spmv_dot<true, tb>), dim3(red_grid(n())), dim3(tb), 0, s,
+                           dev(), n(), p, dinv, Mp, y, a, (int)want_yy, f, part);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
 void VelocityStencil::init(const double *x, const double *b, double *r, double *p, double *rs, double *part,
                            hipStream_t s) const {
-    hipLaunchKernelGGL(k_v5_init, dim3(red_blocks(n())), dim3(BS), 0, s, dev(), n(), x, b, r, p, rs, part);
+    by_block(n(), [&](auto tb) {
+        hipLaunchKernelGGL(k_v5_init<tb>, dim3(red_grid(n())), dim3(tb), 0, s, dev(), n(), x, b, r, p, rs, part);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 
@@ -593,7 +610,10 @@ void launch_p5_sweep2(const P5Dev &A, double omega, const double *x, const doubl
 
 void launch_p5_wdot(const P5Dev &A, const double *r, double *part, hipStream_t s) {
     if (!A.dx || !A.dy) throw Error("the constant mode needs the cell widths of the stencil operator", ERR_ARGUMENT);
-    hipLaunchKernelGGL(k_p5_wdot, dim3(red_blocks((long)A.nx * A.ny)), dim3(BS), 0, s, A, r, part);
+    const long n = (long)A.nx * A.ny;
+    by_block(n, [&](auto tb) {
+        hipLaunchKernelGGL(k_p5_wdot<tb>, dim3(red_grid(n)), dim3(tb), 0, s, A, r, part);
+    });
     CUIBM_LAUNCH_CHECK();
 }
 

@@ -48,7 +48,7 @@ Bicgstab::Bicgstab(int n) : n_(n) {
         ws += st;
     }
     part_ = ws;
-    sc_ = ws + 2 * RED_GRID;
+    sc_ = ws + 4 * (size_t)red_parts(n);
     CUIBM_HIP(hipHostMalloc((void **)&host_sc_, SC_COUNT * sizeof(double), hipHostMallocDefault));
     pinned_ = true;
 }
@@ -60,7 +60,7 @@ Bicgstab::Bicgstab(int n, double *ws, double *host_sc) : n_(n), host_sc_(host_sc
         ws += st;
     }
     part_ = ws;
-    sc_ = ws + 2 * RED_GRID;
+    sc_ = ws + 4 * (size_t)red_parts(n);
 }
 
 Bicgstab::~Bicgstab() {
@@ -70,15 +70,13 @@ Bicgstab::~Bicgstab() {
 SolveStat Bicgstab::solve(const LinOp &A, double *x, const double *b, Preconditioner &M, double rtol,
                           int maxit, hipStream_t s) {
     if (A.n() != n_) throw Error("BiCGSTAB workspace size mismatch", ERR_ARGUMENT);
-    const int n = n_, np = red_blocks(n);
-    // small systems: every reduction is finished by the kernel that uses it (FinArgs), from the
-    // half of the partials that this kernel does not write
-    const bool fused = np <= FUSE_PARTS;
-    double *sc = sc_, *part0 = part_, *part1 = fused ? part_ + FUSE_PARTS : part_;
+    const int n = n_, np = red_parts(n);
+    // a reduction is finished by the kernel that uses it (FinArgs), from the half of the partials
+    // that this kernel does not write
+    double *sc = sc_, *part0 = part_, *part1 = part_ + 2 * (size_t)np;
     const double *diag = M.diagonal();
     int par = 0;  // parity of the iteration since the last (re)start
-    auto args = [&](const double *part) { return FinArgs{fused ? part : nullptr, np, sc, par, maxit}; };
-    auto finish = [&](const double *part, int op) { launch_bicg_finish(part, np, op, args(nullptr), s, rtol); };
+    auto args = [&](const double *part) { return FinArgs{part, np, sc, par, maxit}; };
     SolveStat st;
     auto fetch = [&]() {  // the scalar block: one small copy, one sync
         CUIBM_HIP(hipMemcpyAsync(host_sc_, sc, SC_COUNT * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -87,7 +85,7 @@ SolveStat Bicgstab::solve(const LinOp &A, double *x, const double *b, Preconditi
     auto start = [&](int op) {  // r = b - A x, rs = p = r; clears the stop codes
         par = 0;
         A.init(x, b, r_, p_, rs_, part0, s);
-        finish(part0, op);
+        launch_bicg_finish(op, args(part0), s, rtol);
     };
     // the first half of iteration k (through s, and the test on ||s|| if `test`), then the second
     // half. A preconditioner that forms weighted sums of its input gets them from the kernels
@@ -106,9 +104,8 @@ SolveStat Bicgstab::solve(const LinOp &A, double *x, const double *b, Preconditi
             else M.apply(p_, Mp_, s);
             A.spmv_dot(Mp_, AMp_, rs_, false, part0, s);
         }
-        if (!fused) finish(part0, FIN_ALPHA);
         launch_bicg_s(n, r_, AMp_, s_, args(part0), part1, s, wp);
-        if (test) finish(part1, FIN_SS);
+        if (test) launch_bicg_finish(FIN_SS, args(part1), s);
     };
     auto half2 = [&](bool tested) {
         const double *stop = sc + (tested ? (int)SC_STOPS : sc_stop(par));  // FIN_SS hands the other on
@@ -121,14 +118,12 @@ SolveStat Bicgstab::solve(const LinOp &A, double *x, const double *b, Preconditi
             else M.apply(s_, Ms_, s);
             A.spmv_dot(Ms_, AMs_, s_, true, part0, s);
         }
-        if (!fused) finish(part0, FIN_OMEGA);
         launch_bicg_xr(n, x, Mp_, Ms_, r_, s_, AMs_, rs_, args(part0), part1, s);
-        if (!fused) finish(part1, FIN_BETA);
         launch_bicg_p(n, p_, r_, AMp_, args(part1), s, wp);
         p_weighted = wp != nullptr;
         par ^= 1;
     };
-    const bool test_early = !(diag && fused);  // ||s|| is tested before the second product (else in it)
+    const bool test_early = !diag;  // ||s|| is tested before the second half (else in its product)
     start(FIN_INIT);
     double tol = 0, rn = 0, rn0 = 0, rn_ref = 0;
     // with an earlier solve to go by, iterations are queued before the first read-back
@@ -185,7 +180,7 @@ SolveStat Bicgstab::solve(const LinOp &A, double *x, const double *b, Preconditi
                     fetch();
                     const int h = (int)host_sc_[SC_STOPS], c = (int)host_sc_[sc_stop(par)];
                     if (c == 0 && h == STOP_HALF_PENDING) {  // the half-step update alone
-                        launch_bicg_xr(n, x, Mp_, Ms_, r_, s_, AMs_, rs_, FinArgs{nullptr, np, sc, par, maxit}, part1, s);
+                        launch_bicg_xr(n, x, Mp_, Ms_, r_, s_, AMs_, rs_, args(part0), part1, s);
                         code = STOP_HALF;
                     } else if (c != 0 || h != 0) {
                         code = c != 0 ? c : h;

@@ -3,17 +3,32 @@
 #pragma once
 #include <memory>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "dev.hpp"
 
 namespace cuibm {
 
-constexpr int RED_GRID = 2048;  // most blocks of a reducing kernel, and partial sums of one group
-// blocks of the reducing kernels of n unknowns: one block per BS unknowns (a multiple of 8, see
-// xcd_block) up to RED_GRID, which stride over the vector. The partials do not depend on it:
-// blocks without an unknown would add zeros.
-inline int red_blocks(long n) { return (int)std::min<long>(RED_GRID, (n / BS + 8) / 8 * 8); }
+constexpr int RED_GRID = 2048;  // most partial sums of one group
+// A reduction over n unknowns has red_parts(n) partial sums, each of one group of BS threads (a
+// multiple of 8, see xcd_block; groups without an unknown add zeros). Up to FUSE_PARTS of them a
+// group is a block; above, a block of RED_WIDE threads is four groups, so that few enough blocks
+// run for every one of them to sum the partials of the reduction before it (FinArgs). The sums are
+// the same bits either way.
+constexpr int FUSE_PARTS = 512, RED_WIDE = 1024;
+inline __host__ __device__ int red_parts(long n) {
+    const long p = (n / BS + 8) / 8 * 8;
+    return (int)(p < RED_GRID ? p : RED_GRID);
+}
+inline int red_threads(long n) { return red_parts(n) <= FUSE_PARTS ? BS : RED_WIDE; }
+inline int red_grid(long n) { return red_threads(n) == BS ? red_parts(n) : (red_parts(n) + 31) / 32 * 8; }
+// f(block size as a constant) for n unknowns
+template <class F>
+void by_block(long n, F f) {
+    if (red_threads(n) == BS) f(std::integral_constant<int, BS>{});
+    else f(std::integral_constant<int, RED_WIDE>{});
+}
 
 // slots of the device scalar block. SC_STOP is the device-side end of the iteration:
 // 0 running, STOP_* below otherwise; every kernel of the iteration returns at once when
@@ -35,15 +50,13 @@ enum { STOP_CONVERGED = 1, STOP_HALF = 2, STOP_BREAK_HALF = 3, STOP_BREAK_FULL =
 // the iteration count, the tolerance and the half-step record are kept
 enum { FIN_INIT = 0, FIN_ALPHA, FIN_SS, FIN_OMEGA, FIN_BETA, FIN_RESTART };
 
-// The finish of a reduction inside the kernel that uses its result: with `part` the kernel adds
-// the np partials there itself (every block, in k_bicg_finish's order) and one thread stores
-// the scalars, without it a finish launch has. A launch costs 3.5-4 us whatever it does, the
-// sums about 1 us of the consumer for a few hundred partials; beyond FUSE_PARTS every block reading
-// them all costs more (462^2, 840 partials: the x and r update 11.7 us against 5 and a finish of
-// 3, an embedded step 7.8 ms unfused against 8.6). The kernel's own partials go to another half
-// of the buffer. Steps with finishes, Jacobi products and first read-backs fused, before and
-// after: 32^2 cavity 0.29 -> 0.18 ms, 128^2 1.08 -> 0.77, 336^2 cylinder (FP64) 3.1 -> 2.7.
-constexpr int FUSE_PARTS = 512;
+// The finish of a reduction inside the kernel that uses its result: every block adds the np
+// partials in `part` (in k_bicg_finish's order) and one thread stores the scalars. A finish
+// launch of its own costs 3.5-4 us whatever it does, the sums about 1 us of the consumer (with
+// blocks of BS threads, 840 of them on a 462^2 grid, more than the launch: the x and r update 11.7 us
+// against 5). The kernel's own partials go to another half of the buffer. Steps before and after
+// (with Jacobi products and first read-backs fused): 32^2 cavity 0.29 -> 0.18 ms, 128^2 1.08 ->
+// 0.75, 336^2 cylinder (FP64) 3.1 -> 2.6, 1024^2 (FP32 levels) 1.53 -> 1.33.
 struct FinArgs {
     const double *part = nullptr;
     int np = 0;
@@ -69,7 +82,7 @@ void launch_spmv_dot_jacobi(const DCsr<double> &A, const double *dinv, const dou
 void launch_bicg_init(const DCsr<double> &A, const double *x, const double *b, double *r, double *p, double *rs,
                       double *part, hipStream_t s);
 // weights w_i = wx[i % nx] * wy[i / nx] of a preconditioner's input (cell areas), whose
-// RED_GRID partial sums of w_i v_i the kernel producing the input v writes into part
+// red_parts(n) partial sums of w_i v_i the kernel producing the input v writes into part
 struct InputWeights {
     const double *wx = nullptr, *wy = nullptr;
     int nx = 0;
@@ -85,10 +98,9 @@ void launch_bicg_xr(int n, double *x, const double *Mp, const double *Ms, double
 // p = r + beta (p - omega AMp) (after FIN_BETA); with w, also the weighted partials of p
 void launch_bicg_p(int n, double *p, const double *r, const double *AMp, const FinArgs &f, hipStream_t s,
                    const InputWeights *w = nullptr);
-// one block: sums the np partials of each group and updates the scalars of iteration parity
-// f.par; FIN_INIT also forms the tolerance rtol ||b||, FIN_SS and FIN_BETA apply the stopping
-// tests of the monitor and the iteration limit
-void launch_bicg_finish(const double *part, int np, int op, const FinArgs &f, hipStream_t s, double rtol = 0);
+// one block: the finish of a (re)start (FIN_INIT also forms the tolerance rtol ||b||, FIN_RESTART
+// keeps it), or of the half step's stopping test (FIN_SS)
+void launch_bicg_finish(int op, const FinArgs &f, hipStream_t s, double rtol = 0);
 void launch_jacobi_apply(int n, const double *dinv, const double *r, double *z, hipStream_t s,
                          const double *stop = nullptr);
 void launch_diag_inv(const DCsr<double> &A, double *dinv, hipStream_t s);
@@ -396,7 +408,7 @@ class Bicgstab {
     // (256-byte aligned), `host_sc` SC_COUNT host doubles; allocates nothing
     Bicgstab(int n, double *ws, double *host_sc);
     ~Bicgstab();
-    static size_t workspace_doubles(int n) { return 8 * stride(n) + 2 * RED_GRID + SC_COUNT; }
+    static size_t workspace_doubles(int n) { return 8 * stride(n) + 4 * (size_t)red_parts(n) + SC_COUNT; }
     // cusp::krylov::bicgstab + cusp::monitor(b, maxit, rtol) semantics; x is the warm start
     SolveStat solve(const LinOp &A, double *x, const double *b, Preconditioner &M, double rtol, int maxit,
                     hipStream_t s);

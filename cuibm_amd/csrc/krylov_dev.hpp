@@ -29,49 +29,61 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// reduce K values per thread across a 256-thread block; thread 0 gets the sums
-template <int K>
+// reduce K values per thread across each group of BS threads of a block of TB; the group's first
+// thread gets the sums
+template <int K, int TB = BS>
 __device__ __forceinline__ void block_sum(double (&v)[K]) {
-    __shared__ double sh[K][BS / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    __shared__ double sh[K][TB / 64];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, w0 = wid & ~3;
 #pragma unroll
     for (int k = 0; k < K; k++) v[k] = wave_sum(v[k]);
     if (lane == 0)
 #pragma unroll
         for (int k = 0; k < K; k++) sh[k][wid] = v[k];
     __syncthreads();
-    if (threadIdx.x == 0)
+    if (threadIdx.x % BS == 0)
 #pragma unroll
-        for (int k = 0; k < K; k++) v[k] = (sh[k][0] + sh[k][1]) + (sh[k][2] + sh[k][3]);
+        for (int k = 0; k < K; k++) v[k] = (sh[k][w0] + sh[k][w0 + 1]) + (sh[k][w0 + 2] + sh[k][w0 + 3]);
 }
 
-// the totals of NG groups of at most FUSE_PARTS partials in every thread of a 256-thread block,
-// added as k_bicg_finish's 1024 threads add them (each wavefront stands for four of its 16), so
-// fused and separate finishes give the same bits
-template <int NG>
+// the thread's group of a reduction (see red_parts) in block blk, and its index in the group
+template <int TB>
+__device__ __forceinline__ int red_group(int blk) {
+    return TB == BS ? blk : blk * (TB / BS) + (int)threadIdx.x / BS;
+}
+__device__ __forceinline__ int red_lane() { return threadIdx.x % BS; }
+
+// the totals of NG groups of partials in every thread of a block of TB threads, added as
+// k_bicg_finish's 1024 threads add them (a wavefront of a smaller block stands for several of its
+// 16), so fused and separate finishes give the same bits. A small block has at most FUSE_PARTS.
+template <int NG, int TB>
 __device__ __forceinline__ void finish_sums(const FinArgs &f, double (&tot)[2]) {
+    constexpr int PER = TB == RED_WIDE ? 1 : FUSE_PARTS / TB, NW = TB / 64;
     __shared__ double sh[NG][16];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    double v[NG][4];
+    double v[NG][PER];
 #pragma unroll
     for (int g = 0; g < NG; g++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int k = (int)threadIdx.x + 256 * j;
-            v[g][j] = k < f.np ? f.part[g * RED_GRID + k] : 0.0;
+        for (int j = 0; j < PER; j++) {
+            const int k = (int)threadIdx.x + TB * j;
+            const double *p = f.part + (size_t)g * f.np;
+            v[g][j] = k < f.np ? p[k] : 0.0;
+            if (TB == RED_WIDE && k + RED_WIDE < f.np) v[g][j] += p[k + RED_WIDE];
         }
 #pragma unroll
     for (int g = 0; g < NG; g++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < PER; j++) {
             const double t = wave_sum(v[g][j]);
-            if (lane == 0) sh[g][wid + 4 * j] = t;
+            if (lane == 0) sh[g][wid + NW * j] = t;
         }
     __syncthreads();
 #pragma unroll
     for (int g = 0; g < NG; g++) {
         double t = 0;
-        for (int w = 0; w < 16; w++) t += sh[g][w];
+#pragma unroll
+        for (int w = 0; w < NW * PER; w++) t += sh[g][w];
         tot[g] = t;
     }
 }

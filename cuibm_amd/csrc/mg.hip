@@ -487,7 +487,7 @@ struct TensorMg::Levels {
         c.alloc(1);
         launch_fill(c.p(), 0.0, 1, s);
         P.part = part.p();
-        P.npart = red_blocks((long)nx * ny);
+        P.npart = red_parts((long)nx * ny);
         P.c = c.p();
         // Chebyshev weights of three sweeps on [lmax / 10, lmax], lmax = 2 >= the largest
         // eigenvalue of D^-1 A. Iterations on the 336^2, 498^2 and 1024^2 cylinders at their

@@ -6,8 +6,8 @@
 //   [0, stride)            x, staged from the caller's host vector
 //   [stride, 2 stride)     b, staged likewise
 //   [2 stride, 3 stride)   D^-1 of the Jacobi preconditioner
-//   [3 stride, ...)        the BiCGSTAB workspace: 8 vectors, 2 x 2048 reduction
-//                          partials, the 16-double scalar block
+//   [3 stride, ...)        the BiCGSTAB workspace: 8 vectors, up to 4 x 1032
+//                          reduction partials, the 16-double scalar block
 // Each GPU holds its own copy of the array at its own address, looked up once per device
 // with hipGetSymbolAddress; host code passes only that address to kernels and copies.
 // Calls on one GPU share the array, so calls that overlap on one GPU race.
@@ -19,7 +19,9 @@
 namespace cuibm {
 
 static_assert(NOALLOC_MAX_N % 32 == 0, "stride of the largest system must equal NOALLOC_MAX_N");
-constexpr size_t NOALLOC_DOUBLES = 3 * (size_t)NOALLOC_MAX_N + 8 * (size_t)NOALLOC_MAX_N + 2 * RED_GRID + SC_COUNT;
+// two groups of partials of the largest system, in two halves (red_parts(2^18) = 1032)
+constexpr size_t NOALLOC_PARTS = 4 * (NOALLOC_MAX_N / 256 + 8);
+constexpr size_t NOALLOC_DOUBLES = 3 * (size_t)NOALLOC_MAX_N + 8 * (size_t)NOALLOC_MAX_N + NOALLOC_PARTS + SC_COUNT;
 
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
 
@@ -59,7 +61,7 @@ SolveStat bicgstab_noalloc(const DCsr<double> &A, double *x, const double *b, in
     double *dx = ws, *db = ws + st, *dinv = ws + 2 * st, *kws = ws + 3 * st;
     // the reduction partials and the scalar block start from zero on every call (the
     // array keeps the previous call's contents); a fill kernel, not a memset node
-    launch_fill(kws + 8 * st, 0.0, 2 * RED_GRID + SC_COUNT, s);
+    launch_fill(kws + 8 * st, 0.0, 4 * red_parts(n) + SC_COUNT, s);
     CUIBM_HIP(hipMemcpyAsync(dx, x, n * sizeof(double), hipMemcpyHostToDevice, s));
     CUIBM_HIP(hipMemcpyAsync(db, b, n * sizeof(double), hipMemcpyHostToDevice, s));
     double host_sc[SC_COUNT] = {};

@@ -488,19 +488,16 @@ std::vector<double> NavierStokesSolver::poissonIterationLaunches() const {
     const AmgPrecond *a = dynamic_cast<const AmgPrecond *>(PC2.get());
     if (!a) return L;
     const std::vector<double> vc = a->launch_bytes();
-    const double n = op2->n(), spmv = op2->spmv_bytes(), fin = 16.0 * RED_GRID;
-    // half 1: z = M p, y = A z with <rs, y>, finish, s = r - alpha y with <s, s>, finish
+    const double n = op2->n(), spmv = op2->spmv_bytes();
+    // half 1: z = M p, y = A z with <rs, y>, s = r - alpha y with <s, s>, the half step's test
     L.insert(L.end(), vc.begin(), vc.end());
     L.push_back(spmv + 8 * n);
-    L.push_back(fin);
     L.push_back(3 * 8 * n);
-    L.push_back(fin);
-    // half 2: z = M s, t = A z with <t, s>, <t, t>, finish, x and r with their dots, finish, p
+    L.push_back(8.0 * red_parts((long)n));
+    // half 2: z = M s, t = A z with <t, s>, <t, t>, x and r with their dots, p
     L.insert(L.end(), vc.begin(), vc.end());
     L.push_back(spmv + 8 * n);
-    L.push_back(fin);
     L.push_back(8 * 8 * n);
-    L.push_back(fin);
     L.push_back(4 * 8 * n);
     return L;
 }

@@ -93,7 +93,7 @@ class VelocityStencil : public LinOp {
 void launch_p5_pre(const P5Dev &A, double omega, const double *b, double *x2, double *r, hipStream_t s,
                    KernelProbe *probe = nullptr);
 void launch_p5_sweep2(const P5Dev &A, double omega, const double *x, const double *b, double *xo, hipStream_t s);
-// red_blocks(n) partial sums of w_i r_i (w = cell areas), for the constant mode of a
+// red_parts(n) partial sums of w_i r_i (w = cell areas), for the constant mode of a
 // multigrid input (mg.hpp); returns at once while the Krylov solve's stop code is set
 void launch_p5_wdot(const P5Dev &A, const double *r, double *part, hipStream_t s);
 // one sweep xn = x + omega D^-1 (b - A x) (timing of the finest-level smoother)

@@ -272,7 +272,7 @@ int cuibm_bicgstab(cuibm_csr *A, double *x, const double *b, int precond, int am
  * The same solve as cuibm_bicgstab with precond 0 (NONE) or 1 (DIAGONAL), whose device
  * buffers (the staged x and b, the Jacobi diagonal, the eight BiCGSTAB vectors, the
  * reduction partials and the scalar block) all live in one library-owned device array
- * of 11 * 2^18 + 4112 doubles (23.1 MB), one per GPU, held until the process ends.
+ * of 11 * 2^18 + 4144 doubles (23.1 MB), one per GPU, held until the process ends.
  * Allocates nothing (no hipMalloc, hipFree or pinned host memory). n above 262144
  * (2^18) returns CUIBM_ERR_ARGUMENT; precond 2 returns CUIBM_ERR_UNSUPPORTED (an AMG
  * hierarchy is allocated). Every call on one GPU shares that array, so calls that
