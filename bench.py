@@ -5,10 +5,10 @@ Workload: impulsively started circular cylinder at Re=550 (case
 ``cuibm_amd/cases/cylinderRe550_1024_luo``): D=1 at the origin, [-15,15]^2 with
 h=0.005 on [-0.6,0.6]^2 stretched by 1.008178 to 1024x1024 cells, Luo external
 ghost-node IBM with 628 body points, dt=0.0025. Velocity solve: BiCGSTAB + Jacobi,
-rtol 1e-9. Poisson solve: FP64 BiCGSTAB, rtol 1e-9, preconditioned by the
-smoothed-aggregation V-cycle (2+2 Jacobi sweeps, omega 0.8) run in FP32 (matrix values,
-level vectors and smoother arithmetic), with the operator's pinned constant mode removed
-and restored in FP64 around it (the headline "mixed" form); the outer residual, the
+rtol 1e-9. Poisson solve: FP64 BiCGSTAB, rtol 1e-9, preconditioned by a
+multigrid V-cycle (width-merged grids, 3+3 Chebyshev-weighted Jacobi sweeps, a direct level)
+run in FP32 (level vectors and smoother arithmetic), with the operator's pinned constant
+mode removed and restored in FP64 around it (the headline "mixed" form); the outer residual, the
 Krylov dot products and the projection stay FP64. The same steps are also run with an
 FP64 hierarchy and with FP64 CSR operators everywhere, and the drag coefficients of the
 forms are compared.
@@ -32,7 +32,7 @@ about 55 steps in this method (GPU and CPU restatement alike); the default windo
 (steps 6-45) lies before that.
 
 Prints one JSON line. ``roofline`` reports the dominant kernel of the step (the
-fused finest-level pre-smoothing + residual kernel of the Poisson V-cycle, one per
+fused finest-level pre-smoothing + restricted residual kernel of the Poisson V-cycle, one per
 V-cycle and two V-cycles per BiCGSTAB iteration), timed with a HIP start/stop event
 pair attached to each of its launches (hipExtLaunchKernel, which stamps the kernel's
 own begin and end) over a few live time steps of a second instance of the same form,
@@ -504,7 +504,7 @@ def main():
         "data": "synthetic",
         "config": {
             "workload": "cylinderRe550_1024_luo: Re=550 cylinder, 1024x1024 stretched MAC grid, Luo external "
-                        "IBM, dt=0.0025; Poisson FP64 BiCGSTAB rtol 1e-9 preconditioned by an FP32 SA-AMG V-cycle "
+                        "IBM, dt=0.0025; Poisson FP64 BiCGSTAB rtol 1e-9 preconditioned by an FP32 multigrid V-cycle "
                         "(values, vectors, smoothers) with FP64 removal of the pinned constant mode; velocity FP64 "
                         "BiCGSTAB+Jacobi rtol 1e-9",
             "grid": "1024x1024",

@@ -438,6 +438,9 @@ __global__ void __launch_bounds__(64 * WV) k_b_fdm(const FdmTask<T> *__restrict_
 
 // Rows per wavefront: 8 rows keep the halo's share at 7 rows in 15; where that leaves under
 // MG_SHORT wavefronts (two per SIMD of the 1024), 4 rows shorten each wavefront's chain instead.
+// A cycle with 8 rows everywhere, 4 everywhere, and this rule: 336^2 (FP32) 44.2, 38.4, 38.3 us;
+// 498^2 (FP64) 72.3, 62.8, 63.1; 1024^2 (FP32) 85.9, 77.1, 78.5, where only the finest
+// level has 8 (about even).
 constexpr int MG_SHORT = 2048;
 int strips(int nx, int w) { return (nx + w - 1) / w; }
 bool short_rows(int nx, int ny) { return (long)strips(nx, DOWN_W) * ((ny + 7) / 8) < MG_SHORT; }

@@ -38,8 +38,11 @@ namespace cuibm {
 
 // Sizes at which a level is solved directly: below the finest level, 224 cells an axis (14 tiles
 // of 16), where three more levels and a dense solve took 28 us of a cycle against 12 for the
-// four products; as the finest level, 320, where the exact inverse saves the Krylov iteration
-// (its products grow as n^3).
+// four products (a cycle with 128, 224, 320: 336^2 46, 38, 28 us; 498^2 59, 52, 46; 1024^2 87, 79,
+// 78, the steps within 1% from 224 up); as the finest level, 320, where the exact inverse saves the
+// Krylov iterations (its products grow as n^3: 25 us at 200^2, 37 at 300^2, 55 at 390^2). The line
+// could lie higher: a 336^2 cylinder's FP32 step takes 0.44 ms solved directly and 0.74 with levels,
+// but from 336^2 on solves are to run on three levels or more, which the tests check.
 constexpr int MG_FDM_MAX = 224, MG_DIRECT_MAX = 320;
 // width threshold of the coarsening, in smallest cells of the level. Time steps of the 1024^2,
 // 498^2 and 336^2 cylinders with 4, 5, 6, 7 (FP32 levels): 1.56, 1.59, 1.47, 1.54 ms; 1.60,
