@@ -131,7 +131,9 @@ struct LockstepBatch::Impl {
     static constexpr int MOST_ITS = 8;
     int last_its[2] = {-1, -1};
     // reliable updates of the Poisson solve (the cases' restart_reduction()): a case whose
-    // residual has fallen by this factor since its last (re)start restarts from b - A x
+    // residual has fallen by this factor since its last (re)start restarts from b - A x, after
+    // every MOST_ITS iterations. The read-backs between follow the slowest case; a restart at one
+    // of them would make a case's iterates depend on its companions.
     double reliable2 = 0.0;  // the factor squared (compared with r.r)
     DArray<int> mask;
     std::vector<int> host_mask;
@@ -224,7 +226,7 @@ struct LockstepBatch::Impl {
             for (int c = 0; c < nc; c++)
                 if (scv(c, op)[SC_STOP] == 0.0) running = true;
             if (!running || it >= maxit) break;
-            if (rel2 > 0) {  // reliable updates of the running cases whose residual fell far enough
+            if (rel2 > 0 && it % MOST_ITS == 0) {  // of the running cases whose residual fell far enough
                 bool any = false;
                 for (int c = 0; c < nc; c++) {
                     const double *v = scv(c, op);
@@ -262,7 +264,7 @@ struct LockstepBatch::Impl {
                 continue;
             }
             int batch = it == 0 ? (last > 0 ? last : 1) : std::max(1, last / 4);
-            batch = std::min({batch, MOST_ITS, maxit - it});
+            batch = std::min({batch, rel2 > 0 ? MOST_ITS - it % MOST_ITS : MOST_ITS, maxit - it});
             for (int j = 0; j < batch; j++, it++) {
                 run(0);
                 run(1);

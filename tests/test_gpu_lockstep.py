@@ -78,3 +78,18 @@ def test_lockstep_refuses_cases_it_does_not_cover(tmp_path):
     with pytest.raises(cuibm_amd.CuibmError) as e:
         cuibm_amd.ensemble_run([paths[0], case("cylinderRe40_small_fadlun")], steps=5, lockstep=True)
     assert e.value.code == -5  # CUIBM_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("tol", ["1e-8", "1e-11"])
+def test_lockstep_restarts_do_not_follow_the_companions(tmp_path, tol):
+    """FP32 levels (more than 320 cells an axis) with reliable updates: a case's drag and lift
+    are the same bits whichever other cases are solved beside it"""
+    paths, cases = ens.write_cases(str(tmp_path), n=4, seed=4, steps=20, edges=(330, 480))
+    assert all(c[0] > 320 for c in cases)
+    run = lambda sel: cuibm_amd.ensemble_run([paths[k] for k in sel], "-amgPrecision", "32", "-poissonTol", tol,
+                                             steps=20, workers=4, lockstep=True)
+    first = run([0])
+    for sel in ([0, 1], [0, 3], [0, 1, 2, 3]):
+        r = run(sel)
+        print(tol, sel, r["cd"][0] - first["cd"][0], r["cl"][0] - first["cl"][0], flush=True)
+        assert r["cd"][0] == first["cd"][0] and r["cl"][0] == first["cl"][0]
