@@ -1275,8 +1275,9 @@ struct BatchDev {
 };
 
 struct BatchAmg::Impl {
-    BatchDev<double, double> d64;  // stored hierarchies
-    std::unique_ptr<BatchMg> mg;   // tensor multigrid
+    BatchDev<double, double> d64;  // the stored hierarchies
+    int stored = 0;                // of the first cases
+    std::unique_ptr<BatchMg> mg;   // tensor multigrid of the others
 };
 
 BatchAmg::BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long> &offP, const BCase *tab_dev,
@@ -1285,18 +1286,19 @@ BatchAmg::BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long>
     if (amg.empty()) throw Error("batched V-cycle without cases", ERR_ARGUMENT);
     const int prec = amg[0]->precision();
     std::vector<TensorMg *> mg;
+    int n = 0;  // stored hierarchies
     for (auto *a : amg) {
         if (a->precision() != prec) throw Error("batched V-cycle: cases of different AMG precisions", ERR_ARGUMENT);
         if (!a->has_stencil_level()) throw Error("batched V-cycle: a case without its stencil finest level", ERR_UNSUPPORTED);
-        if (a->tensor()) mg.push_back(a->tensor());
+        mg.push_back(a->tensor());
+        if (a->tensor()) continue;
+        if (n + 1 != (int)mg.size()) throw Error("batched V-cycle: stored hierarchies must come first", ERR_ARGUMENT);
+        n++;
     }
     if (prec != 64 && prec != 32) throw Error("batched V-cycle: AMG precision 64 or 32", ERR_UNSUPPORTED);
-    if (!mg.empty() && mg.size() != amg.size()) throw Error("batched V-cycle: cases of different hierarchies", ERR_ARGUMENT);
-    if (!mg.empty()) {
-        im_->mg.reset(new BatchMg(mg, offP, tab_host, nblk, s));
-        return;
-    }
-    const int n = (int)amg.size();
+    if (n < (int)amg.size()) im_->mg.reset(new BatchMg(mg, offP, tab_host, nblk, s));
+    im_->stored = n;
+    if (n == 0) return;
     std::vector<long> tcount(n);
     for (int c = 0; c < n; c++) tcount[c] = p5_tiles(tab_host[c].p5.nx, tab_host[c].p5.ny);
     std::vector<const double *> stops(n);
@@ -1305,8 +1307,8 @@ BatchAmg::BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long>
     B.omega = amg[0]->prm_.omega;
     B.tab = tab_dev;
     std::vector<AmgDev<double, double> *> cd;
-    for (auto *a : amg) cd.push_back(&a->im_->d64);
-    B.build(cd, offP, stops, s);
+    for (int c = 0; c < n; c++) cd.push_back(&amg[c]->im_->d64);
+    B.build(cd, std::vector<long>(offP.begin(), offP.begin() + n), stops, s);
     B.tilemap.build(tcount, 1, s);
     B.tiles = B.tilemap.dev();
     CUIBM_HIP(hipStreamSynchronize(s));
@@ -1315,12 +1317,12 @@ BatchAmg::BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long>
 BatchAmg::~BatchAmg() = default;
 
 void BatchAmg::apply(const double *r, double *z, hipStream_t s) {
+    if (im_->stored > 0) im_->d64.apply(r, z, s);
     if (im_->mg) im_->mg->apply(r, z, s);
-    else im_->d64.apply(r, z, s);
 }
 
 double *BatchAmg::weights_part() const { return im_->mg ? im_->mg->weights_part() : nullptr; }
 
-int BatchAmg::levels() const { return im_->mg ? im_->mg->levels() : (int)im_->d64.lv.size(); }
+int BatchAmg::levels() const { return std::max((int)im_->d64.lv.size(), im_->mg ? im_->mg->levels() : 0); }
 
 }  // namespace cuibm

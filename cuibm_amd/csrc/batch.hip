@@ -114,7 +114,6 @@ struct LockstepBatch::Impl {
     DArray<int> solid;
     int nsolid = 0;
     std::unique_ptr<BatchAmg> amg;
-    std::vector<std::unique_ptr<AmgPrecond>> own;  // cases whose solver holds another kind
     // Krylov workspace per operator
     struct Work {
         DArray<double> r, rs, p, Mp, AMp, sv, Ms, AMs, part;
@@ -323,10 +322,12 @@ LockstepBatch::LockstepBatch(const std::vector<NavierStokesSolver *> &cases, hip
             d.velocitySolve.maxIterations != B.maxit1 || d.PoissonSolve.maxIterations != B.maxit2)
             throw Error("lockstep batch: the cases' solver tolerances and limits must agree", ERR_ARGUMENT);
     }
-    // deepest hierarchy first (the batched V-cycle's level prefixes), then largest first
+    // stored hierarchies first, deepest first (BatchDev's prefixes), then largest first
     B.order.resize(B.nc);
     std::iota(B.order.begin(), B.order.end(), 0);
     std::stable_sort(B.order.begin(), B.order.end(), [&](int a, int b) {
+        const bool ta = amg[a]->tensor() != nullptr, tb = amg[b]->tensor() != nullptr;
+        if (ta != tb) return tb;
         const int la = amg[a]->info().levels, lb = amg[b]->info().levels;
         if (la != lb) return la > lb;
         return luo[a]->numP > luo[b]->numP;
@@ -337,17 +338,6 @@ LockstepBatch::LockstepBatch(const std::vector<NavierStokesSolver *> &cases, hip
         L[k] = luo[B.order[k]];
         A[k] = amg[B.order[k]];
         B.solver.push_back(L[k]);
-    }
-    // one kind of hierarchy for the batch: where some cases have mg.hpp's levels and others (small
-    // FP64 grids) a stored one, the others get levels of their own too
-    const bool tensor = std::any_of(A.begin(), A.end(), [](AmgPrecond *a) { return a->tensor() != nullptr; });
-    for (int c = 0; c < B.nc && tensor; c++) {
-        if (A[c]->tensor()) continue;
-        AmgParams p = A[c]->params();
-        p.coarse_max = 0;
-        const P5Dev fine = static_cast<PoissonStencil *>(L[c]->op2.get())->dev();
-        B.own.emplace_back(new AmgPrecond(L[c]->dom->dx, L[c]->dom->dy, L[c]->dt, fine, p, s));
-        A[c] = B.own.back().get();
     }
     // segments
     for (int c = 0; c < B.nc; c++) {

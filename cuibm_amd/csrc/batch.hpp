@@ -116,8 +116,9 @@ class TensorMg;
 // that has it is one launch, the constant mode is carried per case.
 class BatchMg {
   public:
-    // nblk: blocks of each case in the P map, whose partial sums of the weighted input the kernels
-    // that produce the input leave in weights_part()
+    // one entry per case of the batch (mg: null for a case of another kind). nblk: blocks of each
+    // case in the P map, whose partial sums of the weighted input the kernels that produce the
+    // input leave in weights_part()
     BatchMg(const std::vector<TensorMg *> &mg, const std::vector<long> &offP, const std::vector<BCase> &tab_host,
             const std::vector<int> &nblk, hipStream_t s);
     ~BatchMg();
@@ -130,17 +131,17 @@ class BatchMg {
     std::unique_ptr<Impl> im_;
 };
 
-// The cases' own preconditioners as one, all of one precision (64 or 32) and of one kind:
-// mg.hpp's levels (BatchMg), or stored hierarchies: the finest level per case in stencil form
-// (the tile kernels above), the CSR levels concatenated block-diagonally, the dense coarsest
-// solves per case.
+// The cases' own preconditioners as one, all of one precision (64 or 32). The first cases may have
+// stored hierarchies (small FP64 grids, or loose tolerances): the finest level per case in stencil
+// form (the tile kernels above), the CSR levels concatenated block-diagonally, the dense coarsest
+// solves per case. The others have mg.hpp's levels (BatchMg).
 class BatchAmg {
   public:
     BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long> &offP, const BCase *tab_dev,
              const std::vector<BCase> &tab_host, const std::vector<int> &nblk, hipStream_t s);
     ~BatchAmg();
     void apply(const double *r, double *z, hipStream_t s);
-    double *weights_part() const;  // null for stored hierarchies
+    double *weights_part() const;  // null for stored hierarchies alone
     int levels() const;
 
   private:

@@ -362,7 +362,6 @@ class AmgPrecond : public Preconditioner {
     // a new hierarchy). CSR finest level only.
     bool refresh(const DCsr<double> &A, hipStream_t s);
     int precision() const { return prm_.precision; }
-    const AmgParams &params() const { return prm_; }
 
   private:
     friend class BatchAmg;

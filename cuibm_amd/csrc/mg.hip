@@ -877,14 +877,16 @@ BatchMg::BatchMg(const std::vector<TensorMg *> &mg, const std::vector<long> &off
     for (int n : nblk) total += n;
     B.part.alloc(std::max<size_t>(total, 1));
     for (size_t k = 0; k < mg.size(); k++) {
+        const size_t part = first;
+        first += nblk[k];
+        if (!mg[k]) continue;
         const TensorMg &M = *mg[k];
         const double *stop = tab_host[k].scP + SC_STOP;
         auto take = [&](auto &set, const auto &L) {
-            set.add(L, offP[k], stop, B.c.p() + k, B.part.p() + first, nblk[k]);
+            set.add(L, offP[k], stop, B.c.p() + k, B.part.p() + part, nblk[k]);
         };
         if (M.f_) take(B.f, *M.f_);
         else take(B.d, *M.d_);
-        first += nblk[k];
         B.levels = std::max(B.levels, (int)M.sizes().size());
     }
     B.d.finish(s);

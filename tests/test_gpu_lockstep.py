@@ -93,3 +93,17 @@ def test_lockstep_restarts_do_not_follow_the_companions(tmp_path, tol):
         r = run(sel)
         print(tol, sel, r["cd"][0] - first["cd"][0], r["cl"][0] - first["cl"][0], flush=True)
         assert r["cd"][0] == first["cd"][0] and r["cl"][0] == first["cl"][0]
+
+
+def test_lockstep_keeps_the_preconditioner_of_each_case(tmp_path):
+    """an FP64 batch at 1e-10 of cases with stored hierarchies (up to 10000 unknowns) and with
+    multigrid levels, both in two sizes: each case's drag and lift are the bits of a batch of its own"""
+    paths, cases = ens.write_cases(str(tmp_path), n=4, seed=14, steps=20, edges=(80, 125))
+    print("edges", [c[0] for c in cases], flush=True)
+    assert sum(c[0] ** 2 <= 10000 for c in cases) == 2
+    tight = ["-amgPrecision", "64", "-velocityTol", "1e-10", "-poissonTol", "1e-10"]
+    r = cuibm_amd.ensemble_run(paths, *tight, steps=20, workers=4, lockstep=True)
+    for k, path in enumerate(paths):
+        one = cuibm_amd.ensemble_run([path], *tight, steps=20, workers=1, lockstep=True)
+        print(k, r["cd"][k] - one["cd"][0], r["cl"][k] - one["cl"][0], flush=True)
+        assert r["cd"][k] == one["cd"][0] and r["cl"][k] == one["cl"][0]

@@ -104,7 +104,7 @@ def test_coarsest_level_as_asked_for(tmp_path):
 
 def test_lockstep_of_both_kinds(tmp_path):
     """an FP64 batch at 1e-10 of a grid small enough for a stored hierarchy and of larger ones:
-    the batch uses the multigrid levels for all (drag within 1e-8 of the cases alone)"""
+    drag within 1e-8 of the cases alone"""
     paths, cases = ens.write_cases(str(tmp_path), n=4, seed=12, steps=20, edges=(80, 150))
     sizes = [c[0] ** 2 for c in cases]
     assert min(sizes) <= 10000 < max(sizes)
