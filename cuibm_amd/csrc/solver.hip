@@ -158,13 +158,15 @@ static HCsr download_csr(const DCsr<double> &A, hipStream_t s) {
 //    cylinder at 1e-8 (bar 1e-10): u differs from the oracle's by 1.3e-10 after 200 steps and 7e-10
 //    after 400 even where the Poisson solves here are exact, by 2e-15 with the stored hierarchy, at
 //    4.1 ms a step against 1.0. 1024^2 at 1e-9: 7e-11 between hierarchies, 14.7 ms against 1.6;
-//  - up to four times the largest dense level, where p is compared with its weakly pinned constant
-//    (67^2 cylinder at 1e-12: 1.5e-10 against 1e-14).
-// A system of up to coarse_max unknowns is one dense inverse either way.
+//  - up to MG_SMALL unknowns, where p is compared with its weakly pinned constant (67^2 cylinder at
+//    1e-12: 1.5e-10 against 1e-14).
+// A system of up to coarse_max unknowns is one dense inverse either way; coarse_max takes no other
+// part in the choice.
 constexpr double MG_RTOL = 1e-9;
+constexpr int MG_SMALL = 10000;
 static bool tensor_levels(const LinearSolverParams &p, int n, int coarse_max) {
     if (n <= coarse_max) return false;
-    return p.amgPrecision == 32 || (p.tolerance <= MG_RTOL && n > 4 * coarse_max);
+    return p.amgPrecision == 32 || (p.tolerance <= MG_RTOL && n > MG_SMALL);
 }
 
 // `fine` and `dom`, when given: A in stencil form and its grid

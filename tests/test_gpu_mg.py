@@ -17,8 +17,9 @@ import pytest
 import scipy.sparse as sp
 
 import cuibm_amd
+import pyoracle as po
 from cuibm_amd import ensemble as ens
-from helpers import case
+from helpers import case, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -100,6 +101,26 @@ def test_coarsest_level_as_asked_for(tmp_path):
     """-amgCoarseMax bounds the directly solved level"""
     check(write_case(tmp_path, 130, 120, "NAVIER_STOKES_SOLVER"), 64, 10, "-amgCoarseMax", 400)
     check(case("cylinderRe40_luo"), 64, 10, "-poissonTol", "1e-10", "-amgCoarseMax", 3000)
+
+
+def test_coarsest_level_does_not_choose_the_kind():
+    """4489 unknowns to 1e-12 in FP64 keep the stored hierarchy with a small -amgCoarseMax too: the
+    oracle's iterations (33 to 5 with the multigrid levels), to the one that rounding may move"""
+    tol = {"velocityTol": 1e-12, "poissonTol": 1e-12}
+    po.set_amg_coarse_max(400)
+    try:
+        o = po.Oracle(po.read_case(case("cylinderRe40_small_luo"), tol))
+        o.step(3)
+    finally:
+        po.set_amg_coarse_max(0)
+    with cuibm_amd.Solver(case("cylinderRe40_small_luo"), "-velocityTol", "1e-12", "-poissonTol", "1e-12",
+                          "-amgCoarseMax", "400", diagnostics=False) as g:
+        g.initialise()
+        g.step_time(3)
+        d = rel_l2(g.get("p"), o.get("p"))
+        print("p", d, "iterations", g.info()["iter2"], o.info()["iter2"], flush=True)
+        assert abs(g.info()["iter2"] - o.info()["iter2"]) <= 1
+        assert d <= 1e-10
 
 
 def test_lockstep_of_both_kinds(tmp_path):
