@@ -465,7 +465,8 @@ struct TensorMg::Levels {
     FdmTask<T> direct{};
     bool fine_direct = false;
 
-    void build(const std::vector<MgHostLevel> &h, double dt, int centre, bool round32, hipStream_t s) {
+    // `sign`: of the cell areas that weight the partial sums (h has the magnitudes)
+    void build(const std::vector<MgHostLevel> &h, double dt, int centre, bool round32, double sign, hipStream_t s) {
         const size_t n = h.size() - 1;  // smoothed levels
         fine_direct = n == 0;
         const int nx = (int)h[0].dx.size(), ny = (int)h[0].dy.size();
@@ -485,7 +486,7 @@ struct TensorMg::Levels {
             wa += area(centre) * P.ac;
         }
         if (!(wa > 0)) throw Error("the Poisson operator has no pinned cell to deflate", ERR_ARGUMENT);
-        P.inv_wa = 1.0 / wa;
+        P.inv_wa = sign / wa;
         part.alloc(RED_GRID);
         c.alloc(1);
         launch_fill(c.p(), 0.0, 1, s);
@@ -699,14 +700,20 @@ TensorMg::TensorMg(const std::vector<double> &dx, const std::vector<double> &dy,
                    int coarse_max, const double *dx_dev, const double *dy_dev, hipStream_t s) {
     // a small grid is solved directly, in FP64 whatever the precision of the levels would be
     const bool direct = coarse_max <= 0 && std::max(dx.size(), dy.size()) <= (size_t)MG_DIRECT_MAX;
-    const std::vector<MgHostLevel> h = mg_levels(dx, dy, direct ? MG_DIRECT_MAX : MG_FDM_MAX, coarse_max);
+    // an axis that runs downwards has negative widths; the operator holds products of two
+    auto magnitudes = [](std::vector<double> w) {
+        for (double &v : w) v = std::fabs(v);
+        return w;
+    };
+    const double sign = (dx[0] < 0) == (dy[0] < 0) ? 1.0 : -1.0;
+    const std::vector<MgHostLevel> h = mg_levels(magnitudes(dx), magnitudes(dy), direct ? MG_DIRECT_MAX : MG_FDM_MAX, coarse_max);
     for (const MgHostLevel &L : h) sizes_.emplace_back((int)L.dx.size(), (int)L.dy.size());
     if (precision == 32 && h.size() > 1) {
         f_.reset(new Levels<float>);
-        f_->build(h, dt, centre, false, s);
+        f_->build(h, dt, centre, false, sign, s);
     } else {
         d_.reset(new Levels<double>);
-        d_->build(h, dt, centre, precision == 3264 && h.size() > 1, s);
+        d_->build(h, dt, centre, precision == 3264 && h.size() > 1, sign, s);
     }
     w_.nx = (int)dx.size();
     w_.wx = dx_dev;

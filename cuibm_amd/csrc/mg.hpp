@@ -131,7 +131,11 @@ struct AxisModes {
 };
 AxisModes axis_modes(const std::vector<double> &w, double dt);
 
-// the preconditioner of one case; `precision` 64, 32 (levels in FP32) or 3264 (level
+// whether the widths of an axis can be coarsened: finite, none zero, all of one sign (the
+// operator holds products of two widths, so an axis may run downwards)
+bool mg_axis(const std::vector<double> &w);
+
+// the preconditioner of one case, on axes that mg_axis() accepts; `precision` 64, 32 (levels in FP32) or 3264 (level
 // coefficients rounded to FP32, vectors and arithmetic in FP64)
 class TensorMg {
   public:

@@ -78,6 +78,12 @@ std::vector<MgHostLevel> mg_levels(const std::vector<double> &dx, const std::vec
     }
 }
 
+bool mg_axis(const std::vector<double> &w) {
+    return !w.empty() && std::all_of(w.begin(), w.end(), [&](double v) {
+        return std::isfinite(v) && v != 0 && std::signbit(v) == std::signbit(w[0]);
+    });
+}
+
 void axis_couplings(const std::vector<double> &w, double dt, std::vector<double> &next, std::vector<double> &prev) {
     const size_t n = w.size();
     next.assign(n, 0.0);

@@ -13,6 +13,7 @@
 #include <iomanip>
 #include <sstream>
 
+#include "mg.hpp"
 #include "solver.hpp"
 #include "stencil.hpp"
 
@@ -186,7 +187,7 @@ static std::unique_ptr<Preconditioner> make_precond(const LinearSolverParams &p,
             ap.refreshable = !fused_restriction;  // rebuilt every step: keep the symbolic structure
             ap.pad_nx = ap.refreshable ? pad_nx : 0;
             ap.restart = p.restartReduction;
-            if (fine && tensor_levels(p, A.n, coarse_max)) {
+            if (fine && tensor_levels(p, A.n, coarse_max) && mg_axis(dom->dx) && mg_axis(dom->dy)) {
                 ap.coarse_max = p.amgCoarseMax;
                 return std::unique_ptr<Preconditioner>(new AmgPrecond(dom->dx, dom->dy, dt, *fine, ap, s));
             }

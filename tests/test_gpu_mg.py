@@ -24,13 +24,13 @@ from helpers import case, rel_l2
 pytestmark = pytest.mark.gpu
 
 
-def write_case(d, nx, ny, solver, ratio=None, h=None):
-    """a cavity of nx x ny equal cells (solver NAVIER_STOKES_SOLVER), or a cylinder on a grid
-    stretched by `ratio` from spacing h"""
+def write_case(d, nx, ny, solver, ratio=None, h=None, ends=(1.0, 1.0)):
+    """a cavity of nx x ny equal cells from 0 to `ends` (solver NAVIER_STOKES_SOLVER), or a
+    cylinder on a grid stretched by `ratio` from spacing h"""
     if ratio is None:
-        axis = lambda n, m: (f"- direction: {n}\n  start: 0.0\n  mid_h: {1.0 / (m + 0.5)!r}\n  subDomains:\n"
-                             "    - end: 1.0\n      stretchRatio: 1.0\n")
-        dom = axis("x", nx) + axis("y", ny)
+        axis = lambda n, m, e: (f"- direction: {n}\n  start: 0.0\n  mid_h: {e / (m + 0.5)!r}\n  subDomains:\n"
+                                f"    - end: {e!r}\n      stretchRatio: 1.0\n")
+        dom = axis("x", nx, ends[0]) + axis("y", ny, ends[1])
     else:
         axis = lambda n: (f"- direction: {n}\n  start: -15.0\n  mid_h: {h!r}\n  subDomains:\n    - end: -0.6\n"
                           f"      stretchRatio: {ratio!r}\n    - end: 0.6\n      stretchRatio: 1.0\n"
@@ -77,6 +77,15 @@ def check(folder, precision, most, *args):
                                              (101, 100, 64), (320, 320, 64)])
 def test_direct_grids(tmp_path, nx, ny, precision):
     check(write_case(tmp_path, nx, ny, "NAVIER_STOKES_SOLVER"), precision, 0)
+
+
+# axes that run downwards (negative cell widths): the operator, and the iterations, are those of
+# the axes turned round
+@pytest.mark.parametrize("ends", [(-1.0, 1.0), (1.0, -1.0), (-1.0, -1.0)])
+@pytest.mark.parametrize("nx,ny,precision,most", [(101, 100, 64, 0), (57, 64, 32, 0), (342, 333, 64, 10),
+                                                  (321, 17, 32, 16)])
+def test_axes_that_run_downwards(tmp_path, nx, ny, precision, most, ends):
+    check(write_case(tmp_path, nx, ny, "NAVIER_STOKES_SOLVER", ends=ends), precision, most)
 
 
 # FP32 levels restart after every three digits, and each restart finds the modes of the cavity's
