@@ -261,20 +261,18 @@ __global__ void __launch_bounds__(256) k_dense(int n, int ld, const V *__restric
 
 // the dense coarsest solves of several cases in one launch (lockstep batches): case c's
 // inverse, its size and row stride, and its offset in the level vectors
-template <class V>
 struct DenseCase {
-    const V *inv;
+    const double *inv;
     int n, ld;
     long off;
     const double *stop;  // the case's Krylov stop code: the solve is skipped once it is set
 };
 
-template <class V, class X>
-__global__ void __launch_bounds__(256) k_b_dense(const DenseCase<V> *__restrict__ tab, BMapDev m,
-                                                 const X *__restrict__ b, X *__restrict__ x) {
-    const DenseCase<V> &D = tab[m.cs[blockIdx.x]];
-    dense_row<V, X>(D.n, D.ld, D.inv, b + D.off, x + D.off, m.loc[blockIdx.x] * 4 + (threadIdx.x >> 6),
-                    D.stop ? *D.stop : 0.0);
+__global__ void __launch_bounds__(256) k_b_dense(const DenseCase *__restrict__ tab, BMapDev m,
+                                                 const double *__restrict__ b, double *__restrict__ x) {
+    const DenseCase &D = tab[m.cs[blockIdx.x]];
+    dense_row<double, double>(D.n, D.ld, D.inv, b + D.off, x + D.off, m.loc[blockIdx.x] * 4 + (threadIdx.x >> 6),
+                              D.stop ? *D.stop : 0.0);
 }
 
 }  // namespace
@@ -1068,14 +1066,13 @@ bool AmgPrecond::refresh(const DCsr<double> &A, hipStream_t s) {
 
 namespace {
 
-template <class V>
 struct HCat {
     int n = 0;
     std::vector<int> rp{0}, ci;
-    std::vector<V> v;
+    std::vector<double> v;
     // append the rows of src (columns mapped by col), then empty rows up to `rows`
     template <class F>
-    void append(const std::vector<int> &srp, const std::vector<int> &sci, const std::vector<V> &sv, int rows, F col) {
+    void append(const std::vector<int> &srp, const std::vector<int> &sci, const std::vector<double> &sv, int rows, F col) {
         const int sn = (int)srp.size() - 1;
         for (int i = 0; i < sn; i++) {
             for (int k = srp[i]; k < srp[i + 1]; k++) {
@@ -1087,7 +1084,7 @@ struct HCat {
         for (int i = sn; i < rows; i++) rp.push_back((int)ci.size());
         n += rows;
     }
-    void upload(DCsr<V> &d, int ncols, hipStream_t s) const {
+    void upload(DCsr<double> &d, int ncols, hipStream_t s) const {
         // every row pointer and column inside the operator's shape (host check before any launch)
         if ((int)rp.size() != n + 1 || rp.back() != (int)ci.size())
             throw Error("batched V-cycle: inconsistent concatenated row pointers", ERR_GENERIC);
@@ -1100,7 +1097,7 @@ struct HCat {
         d.nnz = (int)ci.size();
         d.rp.upload(rp, s);
         d.ci.upload(ci.empty() ? std::vector<int>{0} : ci, s);
-        d.v.upload(v.empty() ? std::vector<V>{V(0)} : v, s);
+        d.v.upload(v.empty() ? std::vector<double>{0.0} : v, s);
     }
     int lanes() const {
         HCsr h;
@@ -1112,15 +1109,14 @@ struct HCat {
 
 }  // namespace
 
-template <class V, class X>
 struct BatchDev {
     struct Lvl {
         int n = 0, nS = 0;  // padded rows of the present cases, and of the smoothing prefix
-        DCsr<V> A, G, P, R;
+        DCsr<double> A, G, P, R;
         int lanesA = 1, lanesG = 1, lanesP = 1, lanesR = 1;
-        DArray<V> dinv;
-        DArray<X> b, x, xt, r;
-        DArray<DenseCase<V>> dense;
+        DArray<double> dinv;
+        DArray<double> b, x, xt, r;
+        DArray<DenseCase> dense;
         BMap dmap;
         DArray<int> seg;  // the case of each BATCH_PAD-row segment of the level vectors
     };
@@ -1132,7 +1128,7 @@ struct BatchDev {
     double omega = 0.8;
     DArray<const double *> cstop;  // each case's Poisson stop code: the CSR levels skip stopped cases
 
-    void build(const std::vector<AmgDev<V, X> *> &cd, const std::vector<long> &offP,
+    void build(const std::vector<AmgDev<double, double> *> &cd, const std::vector<long> &offP,
                const std::vector<const double *> &stops, hipStream_t s) {
         ncases = (int)cd.size();
         int depth = 0;
@@ -1165,29 +1161,29 @@ struct BatchDev {
         }
         for (int l = 0; l < depth; l++) {
             Lvl &L = lv[l];
-            HCat<V> A, G, P, R;
-            std::vector<V> dinv;
-            std::vector<DenseCase<V>> dense;
+            HCat A, G, P, R;
+            std::vector<double> dinv;
+            std::vector<DenseCase> dense;
             std::vector<long> dcount;
             std::vector<int> dcase;
             int nS = 0;
             for (int c = 0; c < ncases; c++) {
-                AmgDev<V, X> &d = *cd[c];
+                AmgDev<double, double> &d = *cd[c];
                 if ((int)d.lv.size() <= l) continue;
                 const int rows = (int)batch_pad(d.lv[l].n);
                 if ((int)d.lv.size() - 1 == l) {  // this case's coarsest level
-                    dense.push_back(DenseCase<V>{d.coarse_inv.p(), d.nc, d.ld, off[l][c], stops[c]});
+                    dense.push_back(DenseCase{d.coarse_inv.p(), d.nc, d.ld, off[l][c], stops[c]});
                     dcount.push_back(d.nc);
                     continue;
                 }
                 nS = (int)(off[l][c] + rows);
-                AmgLevelDev<V, X> &S = d.lv[l];
+                AmgLevelDev<double, double> &S = d.lv[l];
                 const long o = off[l][c], oc = off[l + 1][c];
                 if (l > 0) {
                     if (S.G.n == 0) throw Error("batched V-cycle: a CSR level without its fused restriction", ERR_UNSUPPORTED);
                     A.append(S.A.rp.to_host(s), S.A.ci.to_host(s), S.A.v.to_host(s), rows, [&](int j) { return (int)(o + j); });
-                    std::vector<V> dv = S.dinv.to_host(s);
-                    dv.resize(rows, V(0));
+                    std::vector<double> dv = S.dinv.to_host(s);
+                    dv.resize(rows, 0.0);
                     dinv.insert(dinv.end(), dv.begin(), dv.end());
                 }
                 const int crow = (int)batch_pad(d.lv[l + 1].n);
@@ -1240,22 +1236,22 @@ struct BatchDev {
 
     void vcycle(size_t l, hipStream_t s) {
         Lvl &L = lv[l];
-        const X w = (X)omega;
+        const double w = omega;
         if (L.nS > 0) {
             Lvl &C = lv[l + 1];
             const double *const *cs = cstop.p();
-            launch_pre2<V, X>(L.lanesA, L.A, L.dinv.p(), L.b.p(), L.xt.p(), w, s, nullptr, L.seg.p(), cs);
-            launch_rres<V, X>(L.lanesG, L.G, L.nS, L.xt.p(), L.b.p(), C.b.p(), s, nullptr, C.seg.p(), cs);
+            launch_pre2<double, double>(L.lanesA, L.A, L.dinv.p(), L.b.p(), L.xt.p(), w, s, nullptr, L.seg.p(), cs);
+            launch_rres<double, double>(L.lanesG, L.G, L.nS, L.xt.p(), L.b.p(), C.b.p(), s, nullptr, C.seg.p(), cs);
             vcycle(l + 1, s);
-            launch_csr_op<V, X, OP_PROLONG>(L.lanesP, L.P, C.x.p(), nullptr, nullptr, L.xt.p(), X(0), s, nullptr,
+            launch_csr_op<double, double, OP_PROLONG>(L.lanesP, L.P, C.x.p(), nullptr, nullptr, L.xt.p(), 0.0, s, nullptr,
                                             L.seg.p(), cs);
-            launch_csr_op<V, X, OP_JACOBI>(L.lanesA, L.A, L.xt.p(), L.b.p(), L.dinv.p(), L.r.p(), w, s, nullptr,
+            launch_csr_op<double, double, OP_JACOBI>(L.lanesA, L.A, L.xt.p(), L.b.p(), L.dinv.p(), L.r.p(), w, s, nullptr,
                                            L.seg.p(), cs);
-            launch_csr_op<V, X, OP_JACOBI>(L.lanesA, L.A, L.r.p(), L.b.p(), L.dinv.p(), L.x.p(), w, s, nullptr,
+            launch_csr_op<double, double, OP_JACOBI>(L.lanesA, L.A, L.r.p(), L.b.p(), L.dinv.p(), L.x.p(), w, s, nullptr,
                                            L.seg.p(), cs);
         }
         if (L.dmap.nblk() > 0) {
-            hipLaunchKernelGGL((k_b_dense<V, X>), dim3(L.dmap.nblk()), dim3(256), 0, s, L.dense.p(), L.dmap.dev(),
+            hipLaunchKernelGGL(k_b_dense, dim3(L.dmap.nblk()), dim3(256), 0, s, L.dense.p(), L.dmap.dev(),
                                L.b.p(), L.x.p());
             CUIBM_LAUNCH_CHECK();
         }
@@ -1263,19 +1259,19 @@ struct BatchDev {
 
     void apply(const double *b, double *x, hipStream_t s) {
         Lvl &F = lv[0], &C = lv[1];
-        const X w = (X)omega;
+        const double w = omega;
         launch_b_p5_pre(tab, tiles, w, b, F.xt.p(), F.r.p(), s);
-        launch_csr_op<V, X, OP_SPMV>(F.lanesR, F.R, F.r.p(), nullptr, nullptr, C.b.p(), X(0), s, nullptr, C.seg.p(),
+        launch_csr_op<double, double, OP_SPMV>(F.lanesR, F.R, F.r.p(), nullptr, nullptr, C.b.p(), 0.0, s, nullptr, C.seg.p(),
                                      cstop.p());
         vcycle(1, s);
-        launch_csr_op<V, X, OP_PROLONG>(F.lanesP, F.P, C.x.p(), nullptr, nullptr, F.xt.p(), X(0), s, nullptr,
+        launch_csr_op<double, double, OP_PROLONG>(F.lanesP, F.P, C.x.p(), nullptr, nullptr, F.xt.p(), 0.0, s, nullptr,
                                         F.seg.p(), cstop.p());
         launch_b_p5_sweep2(tab, tiles, w, F.xt.p(), b, x, s);
     }
 };
 
 struct BatchAmg::Impl {
-    BatchDev<double, double> d64;  // the stored hierarchies
+    BatchDev d64;  // the stored hierarchies
     int stored = 0;                // of the first cases
     std::unique_ptr<BatchMg> mg;   // tensor multigrid of the others
 };
@@ -1303,7 +1299,7 @@ BatchAmg::BatchAmg(const std::vector<AmgPrecond *> &amg, const std::vector<long>
     for (int c = 0; c < n; c++) tcount[c] = p5_tiles(tab_host[c].p5.nx, tab_host[c].p5.ny);
     std::vector<const double *> stops(n);
     for (int c = 0; c < n; c++) stops[c] = tab_host[c].p5.stop;
-    BatchDev<double, double> &B = im_->d64;
+    BatchDev &B = im_->d64;
     B.omega = amg[0]->prm_.omega;
     B.tab = tab_dev;
     std::vector<AmgDev<double, double> *> cd;

@@ -41,11 +41,6 @@ void launch_fill(double *x, double v, long n, hipStream_t s) {
     hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(n)), dim3(BS), 0, s, x, v, n);
     CUIBM_LAUNCH_CHECK();
 }
-void launch_fill_f(float *x, float v, long n, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_fill<float>, dim3(grid_for(n)), dim3(BS), 0, s, x, v, n);
-    CUIBM_LAUNCH_CHECK();
-}
 void launch_fill_i(int *x, int v, long n, hipStream_t s) {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_fill<int>, dim3(grid_for(n)), dim3(BS), 0, s, x, v, n);
@@ -353,7 +348,6 @@ __device__ __forceinline__ void finish_update(int op, const double (&tot)[2], do
                 sc[SC_STOP] = STOP_BREAK_HALF;
             } else if (sqrt(tot[0]) <= tol) {
                 sc[SC_STOP] = STOP_HALF_PENDING;
-                sc[SC_HALFK] = sc[SC_ITS];
             }
             break;
         case FIN_OMEGA: {  // (AMs.s, AMs.AMs); a breakdown leaves omega = 0 so that x stays finite
@@ -551,7 +545,6 @@ __global__ void __launch_bounds__(BS) k_b_finish(int op, const BCase *__restrict
     const double tot[2] = {v[0], v[1]};
     if (fin == FIN_INIT) {
         sc[SC_ITS] = 0.0;
-        sc[SC_HALFK] = -1.0;
         finish_update(fin, tot, sc, 0.0, maxit);
         sc[SC_TOL] = rtol * sqrt(sc[SC_BB]);
         if (sqrt(sc[SC_RR]) <= sc[SC_TOL]) sc[SC_STOP] = STOP_CONVERGED;  // converged at the start

@@ -33,8 +33,8 @@ void by_block(long n, F f) {
 // slots of the device scalar block. SC_STOP is the device-side end of the iteration:
 // 0 running, STOP_* below otherwise; every kernel of the iteration returns at once when
 // it is set, so the host may queue several iterations before reading the block back.
-enum { SC_BB = 0, SC_RHO, SC_ALPHA, SC_OMEGA, SC_BETA, SC_SS, SC_RR, SC_STOP, SC_ITS, SC_HALFK, SC_D0, SC_D1,
-       SC_TOL, SC_RHO2, SC_STOP2, SC_STOPS, SC_COUNT = 16 };
+enum { SC_BB = 0, SC_RHO, SC_ALPHA, SC_OMEGA, SC_BETA, SC_SS, SC_RR, SC_STOP, SC_ITS, SC_D0, SC_TOL,
+       SC_RHO2, SC_STOP2, SC_STOPS, SC_COUNT = 16 };
 // SC_TOL: the absolute tolerance. A single solve keeps rho and the stop code in one slot per
 // parity of the iteration (iteration k reads k & 1 and writes the other) and the half step's stop
 // code in SC_STOPS; SC_D0 holds r.r of the first residual. Batched solves use the first slots.
@@ -47,7 +47,7 @@ enum { STOP_CONVERGED = 1, STOP_HALF = 2, STOP_BREAK_HALF = 3, STOP_BREAK_FULL =
        STOP_HALF_PENDING = 6 };
 // finish-kernel operations
 // FIN_RESTART: a restart (in a batch, of the cases marked in a mask) from the true residual;
-// the iteration count, the tolerance and the half-step record are kept
+// the iteration count and the tolerance are kept
 enum { FIN_INIT = 0, FIN_ALPHA, FIN_SS, FIN_OMEGA, FIN_BETA, FIN_RESTART };
 
 // The finish of a reduction inside the kernel that uses its result: every block adds the np
@@ -67,7 +67,6 @@ struct FinArgs {
 
 // ---- k_blas.hip
 void launch_fill(double *x, double v, long n, hipStream_t s);
-void launch_fill_f(float *x, float v, long n, hipStream_t s);
 void launch_fill_i(int *x, int v, long n, hipStream_t s);
 void launch_copy(double *y, const double *x, long n, hipStream_t s, const double *stop = nullptr);
 void launch_to_float(float *y, const double *x, long n, hipStream_t s);
@@ -325,6 +324,7 @@ class AmgPrecond : public Preconditioner {
     }
     void set_stop(const double *stop) override;
     std::string name() const override {
+        if (tensor()) return "MULTIGRID";
         return prm_.precision == 32 ? "SMOOTHED_AGGREGATION(FP32)"
                                     : prm_.precision == 3264 ? "SMOOTHED_AGGREGATION(FP32 values)" : "SMOOTHED_AGGREGATION";
     }

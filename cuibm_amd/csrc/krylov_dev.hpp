@@ -105,7 +105,6 @@ __device__ __forceinline__ double fin_ss(const double (&tot)[2], double *sc, boo
     if (write) {
         sc[SC_SS] = tot[0];
         sc[SC_STOPS] = code;
-        if (code == STOP_HALF_PENDING) sc[SC_HALFK] = sc[SC_ITS];
     }
     return code;
 }

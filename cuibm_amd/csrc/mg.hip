@@ -57,7 +57,6 @@ __device__ __forceinline__ double wave_total(double v) {
 }
 // the constant mode of the input, the same in every wavefront that forms it
 __device__ __forceinline__ double pin_constant(const MgPins &P) {
-    if (!P.part) return P.c[0];
     double t = 0;
     for (int k = threadIdx.x & 63; k < P.npart; k += 64) t += P.part[k];
     return wave_total(t) * P.inv_wa;
@@ -103,7 +102,7 @@ __device__ __forceinline__ void down_tile(const MgTask<T> &K, const double *__re
         };
         if (near(0, 0) || (K.pins.centre > 0 && near(cI, cJ))) {
             const double c = pin_constant(K.pins);
-            if (tile == 0 && lane == 0 && K.pins.part) K.pins.c[0] = c;  // for the way up
+            if (tile == 0 && lane == 0) K.pins.c[0] = c;  // for the way up
 #pragma unroll
             for (int k = 0; k < N; k++) {
                 if (I == 0 && J0 - 3 + k == 0) raw[k] -= c * K.pins.a0;
@@ -360,7 +359,7 @@ __device__ __forceinline__ void fdm_stage(const FdmTask<T> &K, const double *__r
         const bool p0 = FINE && R == 0, p1 = FINE && K.pins.centre > 0 && cJ / 16 * 16 == R;
         if (p0 || p1) {
             c = pin_constant(K.pins);
-            if (tile == 0 && threadIdx.x == 0 && K.pins.part) K.pins.c[0] = c;  // for the last stage
+            if (tile == 0 && threadIdx.x == 0) K.pins.c[0] = c;  // for the last stage
         }
         if (stopv != 0.0) return;
         const T *f = F.Fx + (size_t)(C + l) * F.px, *br = FINE ? nullptr : K.b + (size_t)(R + l) * F.px;
@@ -680,7 +679,8 @@ struct TensorMg::Levels {
                 hipLaunchKernelGGL(k, g, t, 0, s, direct, b, z);
             }
         };
-        constexpr bool ends = STAGE == 0 || STAGE == 3;  // the others never see the Krylov vectors
+        // stages 1 and 2 never see the Krylov vectors, and FP32 levels are never the finest
+        constexpr bool ends = (STAGE == 0 || STAGE == 3) && std::is_same<T, double>::value;
         if constexpr (ends) fine_direct ? go(k_fdm<T, true, STAGE>) : go(k_fdm<T, false, STAGE>);
         else go(k_fdm<T, false, STAGE>);
         CUIBM_LAUNCH_CHECK();
@@ -775,7 +775,7 @@ std::vector<double> TensorMg::launch_bytes() const {
 
 // ---- lockstep batches: the cycles of many cases as one preconditioner ----
 // Level l of every case that smooths on it is one launch (task table and block map per level),
-// and so are the three products of all directly solved levels.
+// and so is each of the four products of all directly solved levels.
 
 struct BatchMg::Impl {
     template <class T>
@@ -851,10 +851,11 @@ struct BatchMg::Impl {
                     hipLaunchKernelGGL(k, dim3(m.nblk), t, 0, s, tab[f].p(), m, b, z);
                     CUIBM_LAUNCH_CHECK();
                 };
-                f ? go(k_b_fdm<T, true, 0>) : go(k_b_fdm<T, false, 0>);
+                constexpr bool fine = std::is_same<T, double>::value;  // FP32 levels are never the finest
+                f ? go(k_b_fdm<T, fine, 0>) : go(k_b_fdm<T, false, 0>);
                 go(k_b_fdm<T, false, 1>);
                 go(k_b_fdm<T, false, 2>);
-                f ? go(k_b_fdm<T, true, 3>) : go(k_b_fdm<T, false, 3>);
+                f ? go(k_b_fdm<T, fine, 3>) : go(k_b_fdm<T, false, 3>);
             }
             for (size_t l = lv.size(); l-- > 0;)
                 for (int r = 0; r < 2; r++) {

@@ -76,7 +76,7 @@ struct MgPins {
     int centre = -1;             // second pinned cell or -1
     double a0 = 0, ac = 0;       // A 1 at cell 0 and at the centre
     double inv_wa = 0;           // 1 / w^T a
-    const double *part = nullptr;  // npart partial sums of w_i r_i; null: c[0] holds the constant
+    const double *part = nullptr;  // npart partial sums of w_i r_i
     int npart = 0;
     double *c = nullptr;         // the constant of the last input
     // direct solves with two pins: A0^+ (a0 e_0 - (w_0 a0 / w_c) e_centre), and
