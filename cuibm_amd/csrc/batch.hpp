@@ -7,9 +7,9 @@
 // multiple of 64 values so that vector loads stay aligned), and each batched kernel maps
 // its blocks to (case, block within the case) through a block map; the case's geometry,
 // operators and offsets come from a per-case table in device memory. The immersed-
-// boundary stencils and the AMG levels below the finest are concatenated with their
-// indices shifted, so the single-case kernels run on them unchanged; the finest AMG level
-// stays in stencil form per case. Each case keeps its own BiCGSTAB scalars and stop code:
+// boundary stencils and a stored hierarchy's levels below the finest are concatenated with
+// their indices shifted, so the single-case kernels run on them unchanged; its finest level
+// stays in stencil form per case, and so do the levels of mg.hpp. Each case keeps its own BiCGSTAB scalars and stop code:
 // its vector updates stop at its own convergence, and the host loop ends when every case
 // has stopped, so each case's iterate is the one its own solve would stop at.
 #pragma once

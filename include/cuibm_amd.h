@@ -49,9 +49,7 @@ const char *cuibm_last_error(void);
  * -poissonTol, plus -amgPrecision 64|32|3264 (as cuibm_bicgstab's amg_precision; in a
  * solver whose Poisson operator has its stencil form, 32 also carries the pinned constant
  * mode in FP64 around the FP32 V-cycle), -amgCoarseMax N (largest coarsest AMG level, solved
- * directly: 16..6144, default 2500; 60 for a moving embedded body; a stencil-form operator
- * with FP32 levels or a tolerance of 1e-9 or less has levels that follow the cell widths, the
- * coarsest of up to 224 cells an axis unless N says otherwise),
+ * directly: 16..6144, default 2500; 60 for a moving embedded body),
  * -amgRefresh 0|1 (a moving embedded body's Poisson hierarchy is built on a pattern padded
  * around the body's rows and, while each new matrix keeps to it, set up again numerically
  * on the device with its aggregates kept: 1, the default; or built anew on the host every
@@ -60,7 +58,15 @@ const char *cuibm_last_error(void);
  * 0: never; default 1e-3 with the FP32 V-cycle, whose rounding makes it a slightly different
  * map at every apply, and never otherwise), -poissonPreconditioner NAME,
  * -operators csr|stencil, -outputFolder DIR and -output 0|1) and construct the solver
- * (not yet initialised). */
+ * (not yet initialised).
+ *
+ * A Poisson operator in stencil form (plain and LUO solvers) with more unknowns than N has
+ * multigrid levels that follow the cell widths with -amgPrecision 32, and otherwise with a
+ * tolerance of 1e-9 or less and more than 10000 unknowns: the coarsest of up to 224 cells an
+ * axis (and of N unknowns, if -amgCoarseMax is given); a grid of up to 320 cells an axis is then
+ * solved directly in FP64 (unless -amgCoarseMax is given). The others have a stored aggregation
+ * hierarchy. A looser tolerance without -amgPrecision 32 therefore takes longer: about four times
+ * a step at 336^2 and nine times at 1024^2. */
 int cuibm_create(const char *case_folder, int argc, const char *const *argv, cuibm_solver **out);
 
 /* NavierStokesSolver::initialise() (NavierStokesSolver.cu:34-40, luoIBM.cu:27-52,

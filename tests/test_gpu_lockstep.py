@@ -1,13 +1,14 @@
 """Lockstep ensembles on the GPU (cuibm_ensemble_lockstep): every phase of the step is one
 launch over all cases, each case's BiCGSTAB keeping its own scalars and stopping test.
 
-The only difference from running each case alone is the grouping of the dot-product and
-force partial sums (per-case blocks of the batch instead of a fixed grid of 2048 blocks).
+The only differences from running each case alone are the grouping of the dot-product and
+force partial sums (a partial sum per 256 unknowns of the case, at most 2048 of them alone) and,
+with FP32 levels, after how many iterations a restart is considered.
 At solver tolerance 1e-8 that can move a solve's stopping point by an iteration, so drag
 and lift are compared within 1e-7 of the cases run alone with the same AMG precision over
 50 steps of the impulsive start, for the FP32 V-cycle and for the FP64 hierarchy; with
 solves to 1e-12 the FP64 batch's first case agrees with the oracle within 1e-8 after 20
-steps. Graph replays of the solves' iteration blocks equal eager launches bit for bit. Cases
+steps. Graph replays of the solves' half iterations equal eager launches bit for bit. Cases
 that the batch does not cover are refused with an error.
 """
 import numpy as np
@@ -60,7 +61,7 @@ def test_lockstep_fp64_first_case_matches_oracle(tmp_path):
 
 
 def test_lockstep_graphs_equal_eager_launches(tmp_path):
-    """the solves' eight-iteration blocks replayed as captured graphs give the results of
+    """the halves of the solves' iterations replayed as captured graphs give the results of
     the same kernels launched one by one, bit for bit (every step replays each graph several
     times, with the batch's own launches and read-backs between the replays)"""
     steps = 30

@@ -8,8 +8,8 @@ Each solve is checked on the assembled CSR matrix: the residual of the returned 
 one the solve claims, at most rtol ||b|| and the recurrence's rounding, and the solve must take
 no more iterations than the levels are worth: none where the grid is solved directly (the
 first half step already converges), otherwise at most 10, a factor of 10 per iteration over
-the ten digits asked for (they give 20 to 100). A wrong neighbour, weight or aggregate in any
-level costs the rate long before it costs the answer."""
+the ten digits asked for (they give 20 to 100). test_gpu_mg_cycle.py
+compares the values of an iteration."""
 import math
 
 import numpy as np
